@@ -580,8 +580,11 @@ int nyion_q4_quantize(const float* in, int64_t n_rows, int head_dim, uint8_t* ou
  * Replaces swamp_fused_gemv_q4k / fused_gemv_q4k
  * (swamp-kernels/src/fused_gemv_q4k.rs:59-99, 903-927), the Q4_K arm of
  * forward_linear (swamp-engine/src/linear.rs:99-189), with the f32
- * semantics of its scalar path (395-448).  n_cols a positive multiple of
- * 256; W and x 16-byte aligned.  out is written, not accumulated. */
+ * semantics of its scalar path (395-448).  Multiplied on binary16 matrix
+ * cores: a block's integers exactly, x to within 2^-23 of each value (split
+ * into two terms, scaled per 256 values), f32 sums.  n_cols a positive
+ * multiple of 256; W and x 16-byte aligned.  out is written, not
+ * accumulated. */
 int nyion_gemv_q4k(const uint8_t* d_w, const float* d_x, float* d_out, int n_rows, int n_cols,
                    nyion_stream_t stream);
 
@@ -593,7 +596,8 @@ int nyion_gemv_q4k_multi(const uint8_t* const* d_ws, const float* d_x, float* co
                          const int32_t* row_counts, int n_mats, int n_cols,
                          nyion_stream_t stream);
 
-/* batch inputs against one matrix, W read once per four inputs
+/* batch inputs against one matrix, W read once per eight inputs, or per 16 or
+ * 32 of many
  * (fused_gemv_q4k_batched, fused_gemv_q4k.rs:456-485, the Q4_K arm of
  * forward_linear_batch, linear.rs:301-354): x [batch][x_stride] (x_stride
  * >= n_cols, a multiple of 4), out [batch][out_stride] (>= n_rows).  Each

@@ -1,0 +1,96 @@
+"""Q4_K products at the edges of the kernels' tiles (gpu).
+
+Row counts around the 8- and 16-row units and the 32- to 384-row tiles, row
+lengths of 1 to 56 blocks (fewer blocks than a step takes, blocks that do not
+divide among the wavefronts or the four sums, rows whose converted inputs do
+not fit the LDS) and input counts around 8, 16 and 32.  Every input's output is
+checked against the float64 dequantise-then-dot and must equal the single
+call's bit for bit.
+
+Tolerance: inputs are carried to within 2^-23 and products summed in f32, so
+per output |error| <= c 2^-23 sum|w x| with a small c (the sums' roundings add
+up like a random walk); c = 4 is taken, against sum_j of |d scale q x| +
+|dmin min x|, the terms the formula adds.
+"""
+import numpy as np
+import pytest
+import torch
+
+import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    (1, 256, 1), (15, 256, 3), (17, 512, 2), (33, 768, 4), (16, 1280, 5), (4080, 256, 1),
+    (4081, 512, 1), (4097, 768, 2), (300, 2048, 8), (31, 2048, 9), (33, 1792, 16),
+    (65, 2304, 17), (129, 512, 33), (383, 1280, 31), (385, 256, 100), (2050, 512, 200),
+    (40, 5632, 6), (40, 5632, 13), (24, 14336, 1), (24, 14336, 3), (24, 14336, 7),
+    (9, 53248, 2), (9, 53248, 1),
+]
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+@pytest.mark.parametrize("n_rows,n_cols,batch", CASES)
+def test_q4k_tile_edges(gpu, n_rows, n_cols, batch):
+    w = W.q4k_random_weights(n_rows, n_cols, seed=n_rows + n_cols)
+    x = np.random.default_rng(batch).standard_normal((batch, n_cols)).astype(np.float32)
+    x[:, ::7] *= np.float32(1e-4)  # a spread of magnitudes within a block
+    dw, dx = dev(w), dev(x)
+    out = torch.full((batch, n_rows + 3), float("nan"), device="cuda")
+    gpu.gemv_q4k_batched(dw, dx, out, n_rows, n_cols)
+    single = torch.full((n_rows,), float("nan"), device="cuda")
+    singles = []
+    for b in sorted({0, batch // 2, batch - 1}):
+        gpu.gemv_q4k(dw, dx[b].contiguous(), single, n_rows, n_cols)
+        singles.append((b, single.clone()))
+    torch.cuda.synchronize()
+    for b, s in singles:
+        assert torch.equal(out[b, :n_rows], s), b
+    assert torch.isnan(out[:, n_rows:]).all()  # stride padding untouched
+    deq = W.q4k_dequant_np(w, n_rows, n_cols).astype(np.float64).reshape(n_rows, n_cols)
+    ref = x.astype(np.float64) @ deq.T
+    blocks = w.reshape(n_rows, -1, 144)
+    d = blocks[:, :, 0:4].copy().view(np.float16).astype(np.float64)  # d, dmin
+    # at most 15 * 63 d + 63 dmin per weight of the block
+    most = np.repeat(945 * np.abs(d[..., 0]) + 63 * np.abs(d[..., 1]), 256, axis=1)
+    bound = 4 * 2.0**-23 * (np.abs(x).astype(np.float64) @ most.T)
+    got = out[:, :n_rows].cpu().numpy().astype(np.float64)
+    assert np.all(np.abs(got - ref) <= bound), np.max(np.abs(got - ref) / bound)
+
+
+@pytest.mark.parametrize("n_cols,batch", [(512, 1), (512, 4), (512, 20), (14336, 5)])
+def test_q4k_input_extremes(gpu, n_cols, batch):
+    """Zeros, values at either end of f32 and a power-of-two ladder are scaled
+    within their block, blocks and inputs apart from each other; an infinity or
+    a NaN makes its own input's outputs NaN (as inf - inf and 0 * inf do in the
+    formula) and no other's."""
+    n_rows = 37
+    w = W.q4k_random_weights(n_rows, n_cols, seed=5)
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((batch, n_cols)).astype(np.float32)
+    x[0, :256] = 0
+    x[-1, 256:512] = np.float32(1e-38)
+    x[batch // 2, :256] = np.float32(2.0) ** rng.integers(-20, 20, 256)
+    scale = {0: np.float32(1e30), batch - 1: np.float32(1e-30)}.get(batch // 2, np.float32(1))
+    x[batch // 2] *= scale if batch > 2 else np.float32(1)
+    out = torch.empty((batch, n_rows), device="cuda")
+    gpu.gemv_q4k_batched(dev(w), dev(x), out, n_rows, n_cols)
+    torch.cuda.synchronize()
+    deq = W.q4k_dequant_np(w, n_rows, n_cols).astype(np.float64).reshape(n_rows, n_cols)
+    ref = x.astype(np.float64) @ deq.T
+    mag = np.abs(x).astype(np.float64) @ np.abs(deq).T
+    got = out.cpu().numpy().astype(np.float64)
+    assert np.all(np.isfinite(got))
+    assert np.all(np.abs(got - ref) <= 64 * 2.0**-23 * mag + 1e-37)
+    bad = x.copy()
+    bad[0, 3] = np.inf
+    bad[batch - 1, 300] = np.nan
+    gpu.gemv_q4k_batched(dev(w), dev(bad), out, n_rows, n_cols)
+    torch.cuda.synchronize()
+    again = out.cpu().numpy()
+    assert np.isnan(again[0]).all() and np.isnan(again[batch - 1]).all()
+    for b in range(1, batch - 1):
+        assert np.array_equal(again[b], got[b].astype(np.float32)), b
