@@ -20,10 +20,6 @@
 
 namespace nyion {
 
-__device__ __forceinline__ uint32_t f32_to_f16_bits(float x) {
-    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x);
-}
-
 // Quantise one group of `len` (<= 32) elements into 5 words (20 bytes).
 __device__ __forceinline__ void q4_quantize_group(const float* x, int len, uint32_t w[5]) {
     float mx = 0.0f, mn = FLT_MAX;
@@ -45,76 +41,24 @@ __device__ __forceinline__ void q4_quantize_group(const float* x, int len, uint3
     }
 }
 
-// Eight lanes quantise one 32-element group together (lanes 8j .. 8j+7 of a
-// wavefront, every lane active): lane k holds elements 4k .. 4k+3.  The
-// group's max |x| and min x are taken across the eight lanes with DPP (the
-// operations are exact, so the order does not matter), d and dmin are the
-// same f32 values q4_quantize_group computes, and each lane rounds its own
-// four elements.  Returns, in lanes k = 0..4 of the eight, word k of the
-// group's 20 bytes (the header, then the nibble words).
-template <int CTRL>
-__device__ __forceinline__ float q4_dpp(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x), CTRL, 0xf,
-                                                      0xf, false));
-}
-
-__device__ __forceinline__ uint32_t q4_quantize_group8(float4 x) {
-    // from 0 and FLT_MAX as the reference's fold (a NaN element is passed over)
-    float mx = fmaxf(fmaxf(fmaxf(0.0f, fabsf(x.x)), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
-    float mn = fminf(fminf(fminf(FLT_MAX, x.x), x.y), fminf(x.z, x.w));
-    mx = fmaxf(mx, q4_dpp<0xb1>(mx));   // quad_perm [1,0,3,2]
-    mn = fminf(mn, q4_dpp<0xb1>(mn));
-    mx = fmaxf(mx, q4_dpp<0x4e>(mx));   // quad_perm [2,3,0,1]
-    mn = fminf(mn, q4_dpp<0x4e>(mn));
-    mx = fmaxf(mx, q4_dpp<0x141>(mx));  // row_half_mirror: the eight lanes
-    mn = fminf(mn, q4_dpp<0x141>(mn));
-    const float d = (mx > 1e-10f) ? mx / 7.0f : 0.0f;
-    const float dmin = mn;
-    uint32_t bits = 0;  // this lane's four nibbles: bytes 2k and 2k+1 of the nibble area
-    if (d > 1e-10f) {
-        const float e[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float r = roundf((e[i] - dmin) / d);
-            r = fminf(fmaxf(r, 0.0f), 15.0f);
-            bits |= ((uint32_t)r) << (4 * i);
-        }
-    }
-    // nibble word j (1..4) = lanes 2j-2 (low half) and 2j-1 (high half)
-    const uint32_t other =
-        (uint32_t)__builtin_amdgcn_update_dpp((int)bits, (int)bits, 0xb1, 0xf, 0xf, false);
-    const uint32_t pair = bits | (other << 16);  // valid in even lanes
-    const int k = threadIdx.x & 7;
-    const int base = threadIdx.x & ~7;
-    // lane k (1..4) takes the pair word of lane 2k-2 of its group
-    const uint32_t nib = (uint32_t)__shfl((int)pair, base + 2 * (k > 0 ? k - 1 : 0));
-    const uint32_t hdr = f32_to_f16_bits(d) | (f32_to_f16_bits(dmin) << 16);
-    return k == 0 ? hdr : nib;
-}
-
 // ------------------------------------------------------------- kernels
 
 // One thread per (row, head, 4 values): f32 rows, or binary16 rows (F16).
-// With a bf16 source the kernel also records, in the range-status word,
-// whether some V value reaches 65520 in magnitude: the prefill computed
-// P.V with V in binary16, which cannot hold it (checked here, where V is
-// read anyway, instead of in the prefill's inner loop).
 template <bool F16>
 __global__ void kv_write_flat_kernel(WriteArgs a) {
     const int vec = a.head_dim / 4;
     const long long n = (long long)a.rows * a.n_kv_heads * vec;
-    float vmax = 0.f;
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
          i += (long long)gridDim.x * blockDim.x) {
         const int x = (int)(i % vec);
         const int h = (int)((i / vec) % a.n_kv_heads);
         const int r = (int)(i / ((long long)vec * a.n_kv_heads));
-        vmax = fmaxf(vmax, write_kv_vec<F16>(a, r, h, x));
+        write_kv_vec<F16>(a, r, h, x);
     }
-    if (a.k16) report_range(a.status, vmax >= 65520.f, kRangePrefillV);
 }
 
-// The same V range check on its own, for a prefill without a KV write:
+// The V range check of a prefill's history (P.V is computed with V in
+// binary16): whether some |v| reaches 65520, into the range-status word.
 // v [n] bf16 (n a multiple of 4, 8-byte aligned).
 __global__ void v_range_kernel(const uint16_t* v, long long n, unsigned* status) {
     float vmax = 0.f;
@@ -135,7 +79,7 @@ int v_range_check(const uint16_t* v, long long n, hipStream_t stream) {
 }
 
 // Eight lanes per (row, head, group), 4 elements a lane (head_dim a multiple
-// of 32): the f32 or bf16 rows are read contiguously across the wavefront.
+// of 32): the f32 rows are read contiguously across the wavefront.
 // The grid-stride loop runs whole wavefronts (the DPP exchange needs every
 // lane), items past the end store nothing.
 __global__ __launch_bounds__(256) void kv_write_q4x8_kernel(WriteArgs a) {
@@ -151,16 +95,8 @@ __global__ __launch_bounds__(256) void kv_write_q4x8_kernel(WriteArgs a) {
         const int h = (int)((item / groups) % a.n_kv_heads);
         const int r = (int)(item / ((long long)groups * a.n_kv_heads));
         const long long src = ((long long)r * a.n_kv_heads + h) * a.head_dim + 32 * g + 4 * k;
-        float4 kx, vx;
-        if (a.k16) {
-            kx = bf16x4_to_f32(*(const uint2*)(a.k16 + src));
-            vx = bf16x4_to_f32(*(const uint2*)(a.v16 + src));
-        } else {
-            kx = *(const float4*)(a.k + src);
-            vx = *(const float4*)(a.v + src);
-        }
-        const uint32_t wk = q4_quantize_group8(kx);
-        const uint32_t wv = q4_quantize_group8(vx);
+        const uint32_t wk = q4_quantize_group8(*(const float4*)(a.k + src));
+        const uint32_t wv = q4_quantize_group8(*(const float4*)(a.v + src));
         const long long off = ok ? write_row_offset(a, r, h) : -1;
         if (off >= 0 && k < 5) {
             *(uint32_t*)((uint8_t*)a.k_pool + off + kQ4GroupBytes * g + 4 * k) = wk;
@@ -182,23 +118,12 @@ __global__ void kv_write_q4_kernel(WriteArgs a) {
         if (off < 0) continue;
         const long long src = ((long long)r * a.n_kv_heads + h) * a.head_dim + 32 * g;
         const int len = min(32, a.head_dim - 32 * g);
-        float kb[32], vb[32];
-        const float* ks = a.k + (a.k16 ? 0 : src);
-        const float* vs = a.v + (a.k16 ? 0 : src);
-        if (a.k16) {
-            for (int e = 0; e < len; e++) {
-                kb[e] = __uint_as_float((uint32_t)a.k16[src + e] << 16);
-                vb[e] = __uint_as_float((uint32_t)a.v16[src + e] << 16);
-            }
-            ks = kb;
-            vs = vb;
-        }
         uint32_t w[5];
-        q4_quantize_group(ks, len, w);
+        q4_quantize_group(a.k + src, len, w);
         uint32_t* dk = (uint32_t*)((uint8_t*)a.k_pool + off + kQ4GroupBytes * g);
 #pragma unroll
         for (int t = 0; t < 5; t++) dk[t] = w[t];
-        q4_quantize_group(vs, len, w);
+        q4_quantize_group(a.v + src, len, w);
         uint32_t* dv = (uint32_t*)((uint8_t*)a.v_pool + off + kQ4GroupBytes * g);
 #pragma unroll
         for (int t = 0; t < 5; t++) dv[t] = w[t];
@@ -486,8 +411,7 @@ static int launch_write(const WriteArgs& a, int kv_dtype, hipStream_t stream) {
             hipLaunchKernelGGL(kv_write_flat_kernel<true>, dim3(grid_for(n, 256)), dim3(256), 0, stream, a);
         else
             hipLaunchKernelGGL(kv_write_flat_kernel<false>, dim3(grid_for(n, 256)), dim3(256), 0, stream, a);
-    } else if (a.head_dim % 32 == 0 && (a.k16 ? aligned(a.k16, 8) && aligned(a.v16, 8)
-                                                : aligned(a.k, 16) && aligned(a.v, 16))) {
+    } else if (a.head_dim % 32 == 0 && aligned(a.k, 16) && aligned(a.v, 16)) {
         const long long n = (long long)a.rows * a.n_kv_heads * (a.head_dim / 32) * 8;
         hipLaunchKernelGGL(kv_write_q4x8_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream, a);
     } else {
@@ -495,31 +419,6 @@ static int launch_write(const WriteArgs& a, int kv_dtype, hipStream_t stream) {
         hipLaunchKernelGGL(kv_write_q4_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream, a);
     }
     return check_launch("kv write");
-}
-
-// Used by the prefill entry point (prefill_attention.hip).
-int kv_write_impl(void* k_pool, void* v_pool, const int32_t* block_table, int block_tokens,
-                  int num_blocks, int n_kv_heads, int head_dim, int kv_dtype, int start_pos,
-                  int n_tokens, const float* k, const float* v, hipStream_t stream) {
-    int rc;
-    WriteArgs a{};
-    if ((rc = fill_write_args(a, k_pool, v_pool, block_tokens, num_blocks, n_kv_heads, head_dim,
-                              kv_dtype)) != NYION_OK)
-        return rc;
-    if (!block_table || !k || !v) return set_error(NYION_ERR_INVALID, "kv write: null argument");
-    if (start_pos < 0 || n_tokens <= 0)
-        return set_error(NYION_ERR_INVALID, "kv write: start_pos %d, n_tokens %d", start_pos, n_tokens);
-    if (kv_dtype != NYION_KV_Q4_20B && (!aligned(k, 16) || !aligned(v, 16)))
-        return set_error(NYION_ERR_INVALID, "kv write: k/v must be 16-byte aligned");
-    a.tables = block_table;
-    a.positions = nullptr;
-    a.k = k;
-    a.v = v;
-    a.table_stride = (int)(((long long)start_pos + n_tokens + block_tokens - 1) / block_tokens);
-    a.start_pos = start_pos;
-    a.rows = n_tokens;
-    a.per_seq = 0;
-    return launch_write(a, kv_dtype, stream);
 }
 
 int prefill_write_args(WriteArgs& a, void* k_pool, void* v_pool, const int32_t* block_table,
@@ -543,25 +442,8 @@ int prefill_write_args(WriteArgs& a, void* k_pool, void* v_pool, const int32_t* 
     a.start_pos = start_pos;
     a.rows = n_tokens;
     a.per_seq = 0;
-    // the V range check of the prefill rides on the f32 / binary16 write
-    if (kv_dtype != NYION_KV_Q4_20B) a.status = device_status_word();
+    a.status = device_status_word();  // the V range check of the prefill rides on the write
     return NYION_OK;
-}
-
-int kv_write_bf16_impl(void* k_pool, void* v_pool, const int32_t* block_table, int block_tokens,
-                       int num_blocks, int n_kv_heads, int head_dim, int kv_dtype, int start_pos,
-                       int n_tokens, const uint16_t* k, const uint16_t* v, hipStream_t stream) {
-    int rc;
-    WriteArgs a;
-    if ((rc = prefill_write_args(a, k_pool, v_pool, block_table, block_tokens, num_blocks,
-                                 n_kv_heads, head_dim, kv_dtype, start_pos, n_tokens, k, v)) !=
-        NYION_OK)
-        return rc;
-    // a Q4 write has no V range check of its own: the check runs first
-    if (kv_dtype == NYION_KV_Q4_20B &&
-        (rc = v_range_check(v, (long long)n_tokens * n_kv_heads * head_dim, stream)) != NYION_OK)
-        return rc;
-    return launch_write(a, kv_dtype, stream);
 }
 
 }  // namespace nyion
@@ -576,8 +458,24 @@ int nyion_kv_write(void* k_pool, void* v_pool, const int32_t* block_table, int b
     clear_error();
     int rc;
     if ((rc = require_device()) != NYION_OK) return rc;
-    return kv_write_impl(k_pool, v_pool, block_table, block_tokens, num_blocks, n_kv_heads,
-                         head_dim, kv_dtype, start_pos, n_tokens, k, v, (hipStream_t)stream);
+    WriteArgs a{};
+    if ((rc = fill_write_args(a, k_pool, v_pool, block_tokens, num_blocks, n_kv_heads, head_dim,
+                              kv_dtype)) != NYION_OK)
+        return rc;
+    if (!block_table || !k || !v) return set_error(NYION_ERR_INVALID, "kv write: null argument");
+    if (start_pos < 0 || n_tokens <= 0)
+        return set_error(NYION_ERR_INVALID, "kv write: start_pos %d, n_tokens %d", start_pos, n_tokens);
+    if (kv_dtype != NYION_KV_Q4_20B && (!aligned(k, 16) || !aligned(v, 16)))
+        return set_error(NYION_ERR_INVALID, "kv write: k/v must be 16-byte aligned");
+    a.tables = block_table;
+    a.positions = nullptr;
+    a.k = k;
+    a.v = v;
+    a.table_stride = (int)(((long long)start_pos + n_tokens + block_tokens - 1) / block_tokens);
+    a.start_pos = start_pos;
+    a.rows = n_tokens;
+    a.per_seq = 0;
+    return launch_write(a, kv_dtype, (hipStream_t)stream);
 }
 
 int nyion_kv_append_batch(void* k_pool, void* v_pool, const int32_t* block_tables,

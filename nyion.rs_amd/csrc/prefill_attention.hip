@@ -13,7 +13,8 @@
 // staged in LDS feeds eight wavefronts.  Workgroups are numbered so that each XCD
 // (workgroup id mod 8) takes a contiguous run of the (kv head, row block)
 // list: with 8 kv heads every XCD's L2 holds the K/V of one head.  Within a
-// head, row blocks are issued longest-first.
+// head, row blocks are issued longest-first.  A launch too small for that to
+// fill the chip splits the keys of its pairs as well (prefill_split_kernel).
 //
 // Per 64-key tile:
 //   K tile  [64][D] bf16 -> LDS, rows padded by 16 bytes
@@ -35,6 +36,8 @@
 // within the fp16 range (|v| <= 65504).
 #include <math.h>
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "kv_write.hpp"
 
@@ -45,13 +48,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-int kv_write_impl(void* k_pool, void* v_pool, const int32_t* block_table, int block_tokens,
-                  int num_blocks, int n_kv_heads, int head_dim, int kv_dtype, int start_pos,
-                  int n_tokens, const float* k, const float* v, hipStream_t stream);
-int kv_write_bf16_impl(void* k_pool, void* v_pool, const int32_t* block_table, int block_tokens,
-                       int num_blocks, int n_kv_heads, int head_dim, int kv_dtype, int start_pos,
-                       int n_tokens, const uint16_t* k, const uint16_t* v, hipStream_t stream);
 
 struct PrefillArgs {
     const uint16_t* q;  // [N][Hq][D]
@@ -71,12 +67,12 @@ struct PrefillArgs {
     int n_items;   // kv heads x head subsets x row-block groups
     int causal;
     float scale_log2;
-    // the chunk's paged K/V write into f32 or binary16 pools, done by the
-    // kernel (kv_write != 0): each workgroup of head subset 0 writes its own
-    // tokens' rows for its kv head after its attention work
+    // the chunk's paged K/V write, done by the kernel (kv_write != 0): each
+    // workgroup of head subset 0 writes its own tokens' rows for its kv head
+    // after its attention work
     WriteArgs kvw;
     int kv_write;
-    int kv_f16;
+    int kv_dtype;
     int v_check;  // no pools: the same workgroups only check their V rows' range
 };
 
@@ -136,15 +132,15 @@ __device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {
 // One tile's K (or V) in registers between its global loads and its LDS
 // stores (K chunk u: key (tid+NT*u) / (D/8); V unit u: key pair and 8 dims).
 // K is staged one tile ahead of V.
-template <int D>
+template <int D, int THREADS = prefill_threads<D>()>
 struct KStage {
-    static constexpr int NT = prefill_threads<D>();
+    static constexpr int NT = THREADS;
     static constexpr int LOADS = BN * (D / 8) / NT;
     u32x4 k[LOADS];
 };
-template <int D>
+template <int D, int THREADS = prefill_threads<D>()>
 struct VStage {
-    static constexpr int NT = prefill_threads<D>();
+    static constexpr int NT = THREADS;
     static constexpr int UNITS = (BN / 2) * (D / 8) / NT;
     u32x4 v0[UNITS];
     u32x4 v1[UNITS];
@@ -163,11 +159,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t source_rsrc(const uint16_t* ba
 // is read with buffer loads (one per-thread offset, the tile offset in a
 // scalar register); only a tile that reaches outside clamps K rows and
 // zeroes V rows.
-template <int D>
-__device__ __forceinline__ void stage_load_k(KStage<D>& st, const uint16_t* kbase, int tok_stride,
+template <int D, int NT>
+__device__ __forceinline__ void stage_load_k(KStage<D, NT>& st, const uint16_t* kbase, int tok_stride,
                                              int n, int kt, int tid) {
     constexpr int CPR = D / 8;
-    constexpr int STEP = KStage<D>::NT / CPR;  // keys between a thread's chunks
+    constexpr int STEP = NT / CPR;  // keys between a thread's chunks
     if (kt >= 0 && kt + BN <= n) {
         // buffer loads: the source's descriptor and the tile offset in scalar
         // registers, one per-thread 32-bit offset (no per-lane address math)
@@ -175,21 +171,21 @@ __device__ __forceinline__ void stage_load_k(KStage<D>& st, const uint16_t* kbas
         const int off = ((tid / CPR) * tok_stride + 8 * (tid % CPR)) * 2;
         const int t0 = kt * tok_stride * 2, step = STEP * tok_stride * 2;
 #pragma unroll
-        for (int u = 0; u < KStage<D>::LOADS; u++)
+        for (int u = 0; u < KStage<D, NT>::LOADS; u++)
             st.k[u] = __builtin_amdgcn_raw_buffer_load_b128(r, off, t0 + u * step, 0);
         return;
     }
 #pragma unroll
-    for (int u = 0; u < KStage<D>::LOADS; u++) {
+    for (int u = 0; u < KStage<D, NT>::LOADS; u++) {
         const int t = min(max(kt + tid / CPR + u * STEP, 0), n - 1);  // outside: finite, masked
         st.k[u] = *(const u32x4*)(kbase + (long long)t * tok_stride + 8 * (tid % CPR));
     }
 }
 
-template <int D>
-__device__ __forceinline__ void stage_load_v(VStage<D>& st, const uint16_t* vbase, int tok_stride,
+template <int D, int NT>
+__device__ __forceinline__ void stage_load_v(VStage<D, NT>& st, const uint16_t* vbase, int tok_stride,
                                              int n, int kt, int tid) {
-    constexpr int STEP = 8 * (VStage<D>::NT / (BN / 2));  // dims between a thread's units
+    constexpr int STEP = 8 * (NT / (BN / 2));  // dims between a thread's units
     const int t = kt + 2 * (tid % (BN / 2));
     const int d0 = 8 * (tid / (BN / 2));
     if (kt >= 0 && kt + BN <= n) {
@@ -197,14 +193,14 @@ __device__ __forceinline__ void stage_load_v(VStage<D>& st, const uint16_t* vbas
         const int off = ((t - kt) * tok_stride + d0) * 2;
         const int t0 = kt * tok_stride * 2, row = tok_stride * 2;
 #pragma unroll
-        for (int u = 0; u < VStage<D>::UNITS; u++) {
+        for (int u = 0; u < VStage<D, NT>::UNITS; u++) {
             st.v0[u] = __builtin_amdgcn_raw_buffer_load_b128(r, off + 2 * STEP * u, t0, 0);
             st.v1[u] = __builtin_amdgcn_raw_buffer_load_b128(r, off + 2 * STEP * u, t0 + row, 0);
         }
         return;
     }
 #pragma unroll
-    for (int u = 0; u < VStage<D>::UNITS; u++) {
+    for (int u = 0; u < VStage<D, NT>::UNITS; u++) {
         st.v0[u] = t >= 0 && t < n ? *(const u32x4*)(vbase + (long long)t * tok_stride + d0 + STEP * u)
                                    : u32x4{0, 0, 0, 0};
         st.v1[u] = t + 1 >= 0 && t + 1 < n
@@ -216,40 +212,40 @@ __device__ __forceinline__ void stage_load_v(VStage<D>& st, const uint16_t* vbas
 // The tile at key kt (relative to the chunk): keys below 0 come from the
 // history, the rest from the chunk.  kt is uniform, so the selects are
 // scalar and one copy of the loads serves both sources.
-template <int D>
-__device__ __forceinline__ void load_k_tile(KStage<D>& st, const PrefillArgs& a,
+template <int D, int NT>
+__device__ __forceinline__ void load_k_tile(KStage<D, NT>& st, const PrefillArgs& a,
                                             const uint16_t* kbase, const uint16_t* khbase,
                                             int tok_stride, int kt, int tid) {
     const bool hist = kt < 0;
-    stage_load_k<D>(st, hist ? khbase : kbase, tok_stride, hist ? a.n_hist : a.n,
-                    hist ? kt + a.n_hist : kt, tid);
+    stage_load_k<D, NT>(st, hist ? khbase : kbase, tok_stride, hist ? a.n_hist : a.n,
+                        hist ? kt + a.n_hist : kt, tid);
 }
-template <int D>
-__device__ __forceinline__ void load_v_tile(VStage<D>& st, const PrefillArgs& a,
+template <int D, int NT>
+__device__ __forceinline__ void load_v_tile(VStage<D, NT>& st, const PrefillArgs& a,
                                             const uint16_t* vbase, const uint16_t* vhbase,
                                             int tok_stride, int kt, int tid) {
     const bool hist = kt < 0;
-    stage_load_v<D>(st, hist ? vhbase : vbase, tok_stride, hist ? a.n_hist : a.n,
-                    hist ? kt + a.n_hist : kt, tid);
+    stage_load_v<D, NT>(st, hist ? vhbase : vbase, tok_stride, hist ? a.n_hist : a.n,
+                        hist ? kt + a.n_hist : kt, tid);
 }
 
-template <int D>
-__device__ __forceinline__ void stage_store_k(const KStage<D>& st, unsigned char* kslot, int tid) {
+template <int D, int NT>
+__device__ __forceinline__ void stage_store_k(const KStage<D, NT>& st, unsigned char* kslot, int tid) {
     using L = PrefillLds<D>;
     constexpr int CPR = D / 8;
 #pragma unroll
-    for (int u = 0; u < KStage<D>::LOADS; u++) {
-        const int id = tid + KStage<D>::NT * u;
+    for (int u = 0; u < KStage<D, NT>::LOADS; u++) {
+        const int id = tid + NT * u;
         *(u32x4*)(kslot + (id / CPR) * L::KROW + 16 * (id % CPR)) = st.k[u];
     }
 }
 
-template <int D>
-__device__ __forceinline__ void stage_store_v(const VStage<D>& st, unsigned char* vslot, int tid) {
+template <int D, int NT>
+__device__ __forceinline__ void stage_store_v(const VStage<D, NT>& st, unsigned char* vslot, int tid) {
     using L = PrefillLds<D>;
 #pragma unroll
-    for (int u = 0; u < VStage<D>::UNITS; u++) {
-        const int id = tid + VStage<D>::NT * u;
+    for (int u = 0; u < VStage<D, NT>::UNITS; u++) {
+        const int id = tid + NT * u;
         const int key = 2 * (id % (BN / 2));
         const int dc = id / (BN / 2);
         const int col = (key & ~15) + vt_pos(key & 15);  // even: keys key, key+1
@@ -264,6 +260,31 @@ __device__ __forceinline__ void stage_store_v(const VStage<D>& st, unsigned char
             *(uint32_t*)(vslot + (8 * dc + e) * L::VROW + 2 * col) = pack_f16x2(lo, hi);
         }
     }
+}
+
+// A workgroup's share of the chunk's K/V rows, the tokens of its row blocks
+// for its kv head g, into the paged pools (every (token, kv head) by exactly
+// one workgroup), with the V range check the binary16 P.V product needs;
+// without pools, the check alone.
+template <int D>
+__device__ __forceinline__ void write_chunk_rows(const PrefillArgs& a, int g, int hs, int rbg, int tid,
+                                                 int threads) {
+    if ((!a.kv_write && !a.v_check) || hs != 0) return;
+    constexpr int VEC = D / 4;
+    const int r0 = rbg * a.rb_per_wg * 32;
+    const int r1 = min(a.n, r0 + a.rb_per_wg * 32);
+    float vmax = 0.f;
+    for (int i = tid; i < (r1 - r0) * VEC; i += threads) {
+        const int r = r0 + i / VEC, x = i % VEC;
+        if (!a.kv_write)
+            vmax = fmaxf(vmax, v_absmax(*(const uint2*)(a.v + ((long long)r * a.n_kv_heads + g) * D + 4 * x)));
+        else if (a.kv_dtype == NYION_KV_Q4_20B)
+            vmax = fmaxf(vmax, write_kv_q4_vec(a.kvw, r, g, x));  // 8 lanes per group: VEC is a multiple
+        else
+            vmax = fmaxf(vmax, a.kv_dtype == NYION_KV_F16 ? write_kv_vec<true>(a.kvw, r, g, x)
+                                                          : write_kv_vec<false>(a.kvw, r, g, x));
+    }
+    report_range(a.kvw.status, vmax >= 65520.f, kRangePrefillV);
 }
 
 template <int D>
@@ -453,15 +474,15 @@ __global__ __launch_bounds__(prefill_threads<D>(), 512 / prefill_threads<D>()) v
     // registers are in LDS.
     {
         KStage<D> kst1;
-        load_k_tile<D>(kst, a, kbase, khbase, tok_stride, kt0, tid);
-        load_v_tile<D>(vst, a, vbase, vhbase, tok_stride, kt0, tid);
-        if (n_tiles > 1) load_k_tile<D>(kst1, a, kbase, khbase, tok_stride, kt0 + BN, tid);
-        stage_store_k<D>(kst, kslot0, tid);
-        stage_store_v<D>(vst, vslot0, tid);
-        if (n_tiles > 1) stage_store_k<D>(kst1, kslot0 + L::KBYTES, tid);
+        load_k_tile(kst, a, kbase, khbase, tok_stride, kt0, tid);
+        load_v_tile(vst, a, vbase, vhbase, tok_stride, kt0, tid);
+        if (n_tiles > 1) load_k_tile(kst1, a, kbase, khbase, tok_stride, kt0 + BN, tid);
+        stage_store_k(kst, kslot0, tid);
+        stage_store_v(vst, vslot0, tid);
+        if (n_tiles > 1) stage_store_k(kst1, kslot0 + L::KBYTES, tid);
     }
-    if (n_tiles > 2) load_k_tile<D>(kst, a, kbase, khbase, tok_stride, kt0 + 2 * BN, tid);
-    if (n_tiles > 1) load_v_tile<D>(vst, a, vbase, vhbase, tok_stride, kt0 + BN, tid);
+    if (n_tiles > 2) load_k_tile(kst, a, kbase, khbase, tok_stride, kt0 + 2 * BN, tid);
+    if (n_tiles > 1) load_v_tile(vst, a, vbase, vhbase, tok_stride, kt0 + BN, tid);
     __syncthreads();
     floatx16 s0 = scores_half(kslot0, 0);
 
@@ -485,10 +506,10 @@ __global__ __launch_bounds__(prefill_threads<D>(), 512 / prefill_threads<D>()) v
         if (masked) mask_half(s1, kt, 1);
         consume_half(s1, vb);
         // a slot past the last tile is written and never read
-        stage_store_k<D>(kst, kslot(it + 2), tid);
-        stage_store_v<D>(vst, vslot0 + ((it + 1) & 1) * L::VBYTES, tid);
-        if (it + 3 < n_tiles) load_k_tile<D>(kst, a, kbase, khbase, tok_stride, kt + 3 * BN, tid);
-        if (it + 2 < n_tiles) load_v_tile<D>(vst, a, vbase, vhbase, tok_stride, kt + 2 * BN, tid);
+        stage_store_k(kst, kslot(it + 2), tid);
+        stage_store_v(vst, vslot0 + ((it + 1) & 1) * L::VBYTES, tid);
+        if (it + 3 < n_tiles) load_k_tile(kst, a, kbase, khbase, tok_stride, kt + 3 * BN, tid);
+        if (it + 2 < n_tiles) load_v_tile(vst, a, vbase, vhbase, tok_stride, kt + 2 * BN, tid);
         __syncthreads();
     };
     int it = 0;
@@ -526,29 +547,341 @@ __global__ __launch_bounds__(prefill_threads<D>(), 512 / prefill_threads<D>()) v
         }
     }
 
-    // this workgroup's tokens' K/V rows for kv head g into the paged pools
-    // (every (token, kv head) by exactly one workgroup), with the V range
-    // check the binary16 P.V product needs; without pools, the check alone
-    if ((a.kv_write || a.v_check) && hs == 0) {
-        constexpr int VEC = D / 4;
-        const int r0 = rbg * a.rb_per_wg * 32;
-        const int r1 = min(a.n, r0 + a.rb_per_wg * 32);
-        float vmax = 0.f;
-        for (int i = tid; i < (r1 - r0) * VEC; i += prefill_threads<D>()) {
-            const int r = r0 + i / VEC, x = i % VEC;
-            if (!a.kv_write)
-                vmax = fmaxf(vmax, v_absmax(*(const uint2*)(a.v + ((long long)r * a.n_kv_heads + g) * D + 4 * x)));
-            else
-                vmax = fmaxf(vmax, a.kv_f16 ? write_kv_vec<true>(a.kvw, r, g, x)
-                                            : write_kv_vec<false>(a.kvw, r, g, x));
-        }
-        report_range(a.kvw.status, vmax >= 65520.f, kRangePrefillV);
+    write_chunk_rows<D>(a, g, hs, rbg, tid, prefill_threads<D>());
+}
+
+// ---------------------------------------------------------------------------
+// Few work items: the keys split among groups of wavefronts
+// ---------------------------------------------------------------------------
+//
+// A short chunk gives few (kv head, row block) items, and each walks its keys
+// in one chain of tiles at the latency of a wavefront that has its SIMD to
+// itself (1.0 us per 64-key tile at head_dim 64, 1.7 at 128).  Here a workgroup is NG groups of GW
+// wavefronts: the GW wavefronts of a group are (q head, 32-row block) pairs
+// that share K/V tiles, as in prefill_kernel, and the groups take NG equal
+// runs of the keys of the same pairs, each with tile buffers of its own.  Two
+// K and two V^T slots per group fit 160 KB where the pipelined kernel's three
+// and two would not.  At the end the groups' (max, sum, O) are merged through
+// LDS.  The staged V is range-checked on the way (history and chunk), which
+// spares the launch that prefill_kernel needs for a history.
+//
+// Bound: issue.  A step of the two wavefronts of a SIMD takes 1.6 us at
+// head_dim 64, and about a third each with the staging, the exps or the
+// products alone; the phases of the two barely overlap.  Groups of 4 or 1
+// x 4 at 64 spill or leave SIMDs empty.  Taken: 2 x 4 at 64, 4 x 2 at 128.
+template <int D, int GW, int NG>
+struct SplitLds {
+    using L = PrefillLds<D>;
+    static constexpr int GROUP = 2 * (L::KBYTES + L::VBYTES);
+    static constexpr int PART = 64 * (D / 2) * 4 + 2 * 64 * 4;  // one wavefront's O, max and sum
+    static constexpr int BYTES = NG * GROUP > (NG - 1) * GW * PART ? NG * GROUP : (NG - 1) * GW * PART;
+};
+
+template <int D, int GW, int NG>
+__global__ __launch_bounds__(64 * GW * NG) void prefill_split_kernel(PrefillArgs a) {
+    using L = PrefillLds<D>;
+    using S = SplitLds<D, GW, NG>;
+    constexpr int DT = D / 32;  // output dim tiles
+    constexpr int KS = D / 16;  // k-steps of the S product
+    constexpr int NT = 64 * GW;
+    extern __shared__ __attribute__((aligned(16))) unsigned char split_lds[];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int grp = wave / GW, gw = wave % GW;
+    const int tid = (int)threadIdx.x - grp * NT;  // within the group
+    const int j = lane & 31;
+    const int h = lane >> 5;
+
+    const int per = (a.n_items + 7) / 8;
+    const int item = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (item >= a.n_items) return;
+    const int p = item / a.n_rbg;
+    const int rbg = a.n_rbg - 1 - (item - p * a.n_rbg);
+    const int subsets = a.group / a.hw;
+    const int g = p / subsets;
+    const int hs = p - g * subsets;
+    const int head = g * a.group + hs * a.hw + (gw % a.hw);
+    const int row0 = (rbg * a.rb_per_wg + gw / a.hw) * 32;
+    const int wg_row_end = min(a.n, (rbg + 1) * a.rb_per_wg * 32);
+    const int key_end = a.causal ? wg_row_end : a.n;
+    const int n_htiles = (a.n_hist + BN - 1) / BN;
+    const int n_tiles = n_htiles + (key_end + BN - 1) / BN;
+    const int key_lo = -a.n_hist;
+    const int lim = a.causal ? min(row0 + j, a.n - 1) : a.n - 1;
+    // this group's tiles [it0, it1); every group makes `steps` steps
+    const int steps = (n_tiles + NG - 1) / NG;
+    const int it0 = min(grp * steps, n_tiles), it1 = min(it0 + steps, n_tiles);
+    const int kt0 = (it0 - n_htiles) * BN;
+
+    bf16x8 qreg[KS];
+    {
+        // rows past the end repeat the last one and are not stored
+        const uint16_t* qrow = a.q + ((long long)min(row0 + j, a.n - 1) * a.n_heads + head) * D;
+#pragma unroll
+        for (int s = 0; s < KS; s++) qreg[s] = __builtin_bit_cast(bf16x8, *(const uint4*)(qrow + 16 * s + 8 * h));
     }
+    floatx16 o[DT];
+#pragma unroll
+    for (int t = 0; t < DT; t++) o[t] = floatx16{};
+    float mrun = -1e30f, lrun = 0.f, vmax = 0.f;
+
+    const uint16_t* kbase = a.k + (long long)g * D;
+    const uint16_t* vbase = a.v + (long long)g * D;
+    const uint16_t* khbase = a.kh + (long long)g * D;
+    const uint16_t* vhbase = a.vh + (long long)g * D;
+    const int tok_stride = a.n_kv_heads * D;
+    unsigned char* const kslots = split_lds + grp * S::GROUP;
+    unsigned char* const vslots = kslots + 2 * L::KBYTES;
+    KStage<D, NT> kst;
+    VStage<D, NT> vst;
+    // tile it0 + i, clamped to the group's last (with none of its own, the last of all)
+    auto load_tile = [&](int i) __attribute__((always_inline)) {
+        const int kt = kt0 + min(i, it1 - it0 - 1) * BN;
+        load_k_tile(kst, a, kbase, khbase, tok_stride, kt, tid);
+        load_v_tile(vst, a, vbase, vhbase, tok_stride, kt, tid);
+    };
+    auto store_tile = [&](int i) __attribute__((always_inline)) {
+        stage_store_k(kst, kslots + (i & 1) * L::KBYTES, tid);
+        stage_store_v(vst, vslots + (i & 1) * L::VBYTES, tid);
+#pragma unroll
+        for (int u = 0; u < VStage<D, NT>::UNITS; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                vmax = fmaxf(vmax, v_absmax(uint2{vst.v0[u][e], vst.v0[u][e + 1]}));
+                vmax = fmaxf(vmax, v_absmax(uint2{vst.v1[u][e], vst.v1[u][e + 1]}));
+            }
+    };
+    load_tile(0);
+    store_tile(0);
+    // q is waited for here: a wait inside the loop would also drain the loads
+    // of the next tile, every step
+#pragma unroll
+    for (int s = 0; s < KS; s++) asm volatile("" : "+v"(qreg[s]));
+    load_tile(1);
+    __syncthreads();
+
+    // The next tile into the slots that were last read before the barrier
+    // that ended the previous step.  Of the two wavefronts of a SIMD one does
+    // it before its products and one after them, so that one's LDS writes and
+    // conversions run beside the other's matrix work.
+    auto stage = [&](int i) __attribute__((always_inline)) {
+        if (it0 + i + 1 < it1) {
+            store_tile(i + 1);
+            load_tile(i + 2);
+        }
+    };
+    const bool early = wave < GW * NG / 2;
+    for (int i = 0; i < steps; i++) {
+        if (early) stage(i);
+        if (it0 + i < it1) {
+            const int kt = kt0 + i * BN;
+            const unsigned char* ks = kslots + (i & 1) * L::KBYTES;
+            const unsigned char* vs = vslots + (i & 1) * L::VBYTES;
+            const bool masked = (kt + BN > a.n) || (a.causal && kt + BN - 1 > row0) || kt < key_lo;
+            // both halves' scores first: their products run while the first
+            // half's weights are computed, and its P.V while the second's are
+            floatx16 sc[2];
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++) {
+                const unsigned char* kp = ks + (kb * 32 + j) * L::KROW + 16 * h;
+                sc[kb] = floatx16{};
+#pragma unroll
+                for (int s = 0; s < KS; s++)
+                    sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        __builtin_bit_cast(bf16x8, *(const uint4*)(kp + 32 * s)), qreg[s], sc[kb], 0, 0, 0);
+            }
+            if (masked) {
+#pragma unroll
+                for (int kb = 0; kb < 2; kb++) {
+                    const int hi = lim - kt - 32 * kb - 4 * h;
+                    const int lo = key_lo - kt - 32 * kb - 4 * h;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const int c = 8 * (r >> 2) + (r & 3);
+                        sc[kb][r] = c <= hi && c >= lo ? sc[kb][r] : -INFINITY;
+                    }
+                }
+            }
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++) {
+                const floatx16& st = sc[kb];
+                // weights against the running max, which is raised (and they
+                // are redone) only where a lane's sum passes the limit, as in
+                // prefill_kernel
+                halfx8 pa[2];
+                float psum = 0.f;
+                auto exps = [&]() __attribute__((always_inline)) {
+                    float sa = 0.f, sb = 0.f;
+#pragma unroll
+                    for (int t2 = 0; t2 < 2; t2++)
+#pragma unroll
+                        for (int e = 0; e < 8; e += 2) {
+                            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[8 * t2 + e], a.scale_log2, -mrun));
+                            const float p1 =
+                                __builtin_amdgcn_exp2f(__builtin_fmaf(st[8 * t2 + e + 1], a.scale_log2, -mrun));
+                            sa += p0;
+                            sb += p1;
+                            pa[t2][e] = (_Float16)p0;
+                            pa[t2][e + 1] = (_Float16)p1;
+                        }
+                    psum = sa + sb;
+                };
+                exps();
+                if (__any(psum > kPrefillSumLimit)) {
+                    float mt = -INFINITY;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) mt = fmaxf(mt, st[r]);
+                    mt = max_xor32(mt) * a.scale_log2;
+                    const float mnew = fmaxf(mrun, mt);
+                    const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);
+                    mrun = mnew;
+                    lrun *= alpha;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const float ar = __shfl(alpha, 8 * (r >> 2) + 4 * h + (r & 3));
+#pragma unroll
+                        for (int t = 0; t < DT; t++) o[t][r] *= ar;
+                    }
+                    exps();
+                }
+                lrun += psum;
+                const unsigned char* vp = vs + j * L::VROW + 16 * h + 64 * kb;
+#pragma unroll
+                for (int t2 = 0; t2 < 2; t2++)
+#pragma unroll
+                    for (int dt = 0; dt < DT; dt++)
+                        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            pa[t2], __builtin_bit_cast(halfx8, *(const uint4*)(vp + 32 * dt * L::VROW + 32 * t2)),
+                            o[dt], 0, 0, 0);
+            }
+        }
+        if (!early) stage(i);
+        __syncthreads();
+    }
+    report_range(a.kvw.status, vmax >= 65520.f, kRangePrefillV);
+
+    // merge: the other groups' parts in order through LDS
+    const float lt = lrun + __shfl_xor(lrun, 32);
+    float4* const part0 = (float4*)split_lds;
+    constexpr int PART4 = S::PART / 16;
+    if (grp > 0) {
+        float4* pp = part0 + ((grp - 1) * GW + gw) * PART4;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)
+                pp[(dt * 4 + r / 4) * 64 + lane] = float4{o[dt][r], o[dt][r + 1], o[dt][r + 2], o[dt][r + 3]};
+        ((float*)(pp + D * 8))[lane] = mrun;
+        ((float*)(pp + D * 8))[64 + lane] = lt;
+    }
+    __syncthreads();
+    if (grp == 0) {
+        float mall = mrun, lall = 0.f;
+#pragma unroll
+        for (int q = 1; q < NG; q++) mall = fmaxf(mall, ((const float*)(part0 + ((q - 1) * GW + gw) * PART4 + D * 8))[lane]);
+        {
+            const float alpha = __builtin_amdgcn_exp2f(mrun - mall);
+            lall = lt * alpha;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float ar = __shfl(alpha, 8 * (r >> 2) + 4 * h + (r & 3));
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++) o[dt][r] *= ar;
+            }
+        }
+#pragma unroll 1
+        for (int q = 1; q < NG; q++) {
+            const float4* pp = part0 + ((q - 1) * GW + gw) * PART4;
+            const float alpha = __builtin_amdgcn_exp2f(((const float*)(pp + D * 8))[lane] - mall);
+            lall += ((const float*)(pp + D * 8))[64 + lane] * alpha;
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                float ar[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) ar[e] = __shfl(alpha, 8 * (r >> 2) + 4 * h + e);
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++) {
+                    const float4 v = pp[(dt * 4 + r / 4) * 64 + lane];
+                    o[dt][r] = __builtin_fmaf(v.x, ar[0], o[dt][r]);
+                    o[dt][r + 1] = __builtin_fmaf(v.y, ar[1], o[dt][r + 1]);
+                    o[dt][r + 2] = __builtin_fmaf(v.z, ar[2], o[dt][r + 2]);
+                    o[dt][r + 3] = __builtin_fmaf(v.w, ar[3], o[dt][r + 3]);
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int rr = 8 * (r >> 2) + 4 * h + (r & 3);
+            const float lr = __shfl(lall, rr);
+            const int rowg = row0 + rr;
+            if (rowg < a.n) {
+                const float inv = 1.0f / lr;
+                float* orow = a.out + ((long long)rowg * a.n_heads + head) * D;
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++) orow[32 * dt + j] = o[dt][r] * inv;
+            }
+        }
+    }
+    write_chunk_rows<D>(a, g, hs, rbg, (int)threadIdx.x, NT * NG);
 }
 
 }  // namespace nyion
 
 using namespace nyion;
+
+// Work items of a launch whose workgroups (or groups) have `waves` (q head,
+// 32-row block) pairs: 4, 2 or 1 q heads, the largest that divides the group
+// and the wavefront count, the remaining wavefronts more row blocks of them.
+static long long prefill_items(PrefillArgs& a, int waves) {
+    a.hw = std::min(4, waves);
+    while (a.group % a.hw) a.hw /= 2;
+    a.rb_per_wg = waves / a.hw;
+    a.n_rbg = (a.n + 32 * a.rb_per_wg - 1) / (32 * a.rb_per_wg);
+    return (long long)a.n_kv_heads * (a.group / a.hw) * a.n_rbg;
+}
+
+template <int D, int GW, int NG>
+static int launch_prefill_split(PrefillArgs& a, hipStream_t st) {
+    a.n_items = (int)prefill_items(a, GW);
+    constexpr int lds = SplitLds<D, GW, NG>::BYTES;
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    static std::atomic<int> allowed[kMaxDevices];
+    per_device_value(
+        allowed,
+        [] {
+            return hipFuncSetAttribute((const void*)prefill_split_kernel<D, GW, NG>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+        },
+        0);
+    hipLaunchKernelGGL((prefill_split_kernel<D, GW, NG>), dim3(8 * ((a.n_items + 7) / 8)), dim3(64 * GW * NG), lds,
+                       st, a);
+    return check_launch("prefill");
+}
+
+template <int D>
+static int launch_prefill(PrefillArgs& a, hipStream_t st, bool& split) {
+    constexpr int GW = D == 64 ? 2 : 4, NG = D == 64 ? 4 : 2;
+    // Keys split over a workgroup's groups where one such workgroup per CU
+    // holds the launch and every group has two tiles to pipeline.  Measured
+    // (us, whole kernel / split): 32/4 heads of 64, 480 rows 13.3 / 12.6, 384
+    // rows 11.4 / 11.7, 640 rows (320 workgroups, two rounds) 15.3 / 18.1;
+    // 12/12 heads, 768 rows 18.7 / 13.6; 32/8 heads of 128, 256 rows 15.2 /
+    // 14.5, 64 rows 9.8 / 11.4, 1024 rows 34.0 / 27.5, 2048 rows after 2048
+    // 123 / 129; 512 rows after 1536 37.0 / 21.7 (d 64) and 59.0 / 43.3 (d
+    // 128).  With a history the split kernel also saves the launch that
+    // checks its V, which outweighs the merge at any length: one row after
+    // 128 12.5 / 9.7 (d 64) and 13.4 / 10.2 (d 128).
+    constexpr int kCus = 256;
+    const int tiles = (a.n_hist + BN - 1) / BN + (a.n + BN - 1) / BN;
+    split = prefill_items(a, GW) <= kCus && (tiles >= 2 * NG || a.n_hist > 0);
+    if (split) return launch_prefill_split<D, GW, NG>(a, st);
+    const long long items = prefill_items(a, prefill_threads<D>() / 64);
+    if (items > (1LL << 30)) return set_error(NYION_ERR_UNSUPPORTED, "prefill: %lld work items", items);
+    a.n_items = (int)items;
+    hipLaunchKernelGGL(prefill_kernel<D>, dim3(8 * ((a.n_items + 7) / 8)), dim3(prefill_threads<D>()), 0, st, a);
+    return check_launch("prefill");
+}
 
 static int prefill_impl(const uint16_t* q, const uint16_t* k, const uint16_t* v,
                         const uint16_t* k_hist, const uint16_t* v_hist, int n_hist, int n,
@@ -577,12 +910,6 @@ static int prefill_impl(const uint16_t* q, const uint16_t* k, const uint16_t* v,
         (long long)n_hist + n + 2 * BN >= (1LL << 31))
         return set_error(NYION_ERR_UNSUPPORTED, "prefill: history of %d tokens too large", n_hist);
     const int group = n_heads / n_kv_heads;
-    // q heads per workgroup: 4, 2 or 1, the largest that divides the group
-    // (and so also the wavefront count); the remaining wavefronts take more
-    // row blocks of the same heads
-    int hw = 4;
-    while (group % hw) hw /= 2;
-    const int waves = (head_dim == 128 ? 512 : 256) / 64;
     PrefillArgs a{};
     a.q = q;
     a.k = k;
@@ -596,49 +923,31 @@ static int prefill_impl(const uint16_t* q, const uint16_t* k, const uint16_t* v,
     a.n_heads = n_heads;
     a.n_kv_heads = n_kv_heads;
     a.group = group;
-    a.hw = hw;
-    a.rb_per_wg = waves / hw;
-    const int rows_per_wg = 32 * a.rb_per_wg;
-    a.n_rbg = (n + rows_per_wg - 1) / rows_per_wg;
-    const long long items = (long long)n_kv_heads * (group / hw) * a.n_rbg;
-    if (items > (1LL << 30)) return set_error(NYION_ERR_UNSUPPORTED, "prefill: %lld work items", items);
-    a.n_items = (int)items;
     a.causal = causal ? 1 : 0;
     const float sc = scale > 0.f ? scale : 1.0f / sqrtf((float)head_dim);
     a.scale_log2 = sc * 1.4426950408889634f;
     if (k_pool || v_pool) {
         if (!k_pool || !v_pool || !block_table)
             return set_error(NYION_ERR_INVALID, "prefill: KV write needs k_pool, v_pool and block_table");
-        if (kv_dtype == NYION_KV_F32 || kv_dtype == NYION_KV_F16) {
-            if ((rc = prefill_write_args(a.kvw, k_pool, v_pool, block_table, block_tokens, num_blocks,
-                                         n_kv_heads, head_dim, kv_dtype, start_pos, n, k, v)) !=
-                NYION_OK)
-                return rc;
-            a.kv_write = 1;
-            a.kv_f16 = kv_dtype == NYION_KV_F16;
-        }
+        if ((rc = prefill_write_args(a.kvw, k_pool, v_pool, block_table, block_tokens, num_blocks,
+                                     n_kv_heads, head_dim, kv_dtype, start_pos, n, k, v)) != NYION_OK)
+            return rc;
+        a.kv_write = 1;
+        a.kv_dtype = kv_dtype;
     } else {
         a.v_check = 1;
         a.kvw.status = device_status_word();
     }
-    dim3 grid(8 * ((a.n_items + 7) / 8));
     hipStream_t st = (hipStream_t)stream;
-    if (head_dim == 128)
-        hipLaunchKernelGGL(prefill_kernel<128>, grid, dim3(prefill_threads<128>()), 0, st, a);
-    else
-        hipLaunchKernelGGL(prefill_kernel<64>, grid, dim3(prefill_threads<64>()), 0, st, a);
-    if ((rc = check_launch("prefill")) != NYION_OK) return rc;
+    bool split = false;
+    if ((rc = head_dim == 128 ? launch_prefill<128>(a, st, split) : launch_prefill<64>(a, st, split)) != NYION_OK)
+        return rc;
     // V enters the P.V product as binary16: values of magnitude >= 65520 are
     // reported through the status word (the chunk's V by the kernel's own
-    // tail, with or without its f32 / binary16 pool write, or by the Q4
-    // write's check; the history's here)
-    if (n_hist > 0 &&
+    // tail; the history's by the split kernel as it stages it, or here)
+    if (n_hist > 0 && !split &&
         (rc = v_range_check(v_hist, (long long)n_hist * n_kv_heads * head_dim, st)) != NYION_OK)
         return rc;
-    if (!k_pool && !v_pool) return NYION_OK;  // the kernel checked the chunk's V itself
-    if (!a.kv_write)  // 4-bit pools: their own quantising write (with the V range check)
-        return kv_write_bf16_impl(k_pool, v_pool, block_table, block_tokens, num_blocks, n_kv_heads,
-                                  head_dim, kv_dtype, start_pos, n, k, v, st);
     return NYION_OK;
 }
 
