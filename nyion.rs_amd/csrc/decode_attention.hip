@@ -67,6 +67,8 @@ typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 // 16 bytes at 8-byte alignment (binary16 rows): one dwordx4 load
 typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(8)));
+// 8 bytes at 4-byte alignment (4-bit rows): one dwordx2 load
+typedef uint32_t u32x2a __attribute__((ext_vector_type(2), aligned(4)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -625,10 +627,10 @@ struct Q4VOperands {
     uint32_t hi[D / 16][2], lo[D / 16][2], mm[2];
 };
 
-template <int D, bool MASKED>
+// Output dims z = Z0 .. Z1 - 1 (all by default).
+template <int D, bool MASKED, int Z0 = 0, int Z1 = D / 16>
 __device__ __forceinline__ Q4VOperands<D> q4_v_operands(const Tile<D, NYION_KV_Q4_20B>& t, uint32_t mask,
                                                         int kq, uint32_t k6464) {
-    constexpr int DPL = D / 16;
     Q4VOperands<D> o;
     const halfx2 s32 = {(_Float16)0.03125f, (_Float16)0.03125f};
     uint32_t d01 = __builtin_amdgcn_perm(t.vhdr[1], t.vhdr[0], 0x05040100u);
@@ -652,16 +654,16 @@ __device__ __forceinline__ Q4VOperands<D> q4_v_operands(const Tile<D, NYION_KV_Q
     // nibbles are element 2b of the two rows and its high nibbles element
     // 2b + 1, each as binary16 1024 + e after a mask and 0x64 in the high
     // bytes (k6464)
-    constexpr int NBY = DPL / 2;  // nibble bytes per row: 2 at head_dim 64, 4 at 128
+    constexpr int B0 = Z0 / 2, B1 = (Z1 + 1) / 2;  // nibble bytes per row: 2 at head_dim 64, 4 at 128
     const halfx2 k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
-    uint32_t pw[2][NBY];
+    uint32_t pw[2][B1];
 #pragma unroll
     for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int b = 0; b < NBY; b++)
+        for (int b = B0; b < B1; b++)
             pw[p][b] = __builtin_amdgcn_perm(t.v[2 * p + 1], t.v[2 * p], 0x0c000c00u | ((4u + b) << 16) | (uint32_t)b);
 #pragma unroll
-    for (int z = 0; z < DPL; z++) {  // element z: nibble z of the lane's word
+    for (int z = Z0; z < Z1; z++) {  // element z: nibble z of the lane's word
         const int b = z >> 1;
         const uint32_t n01 = (((z & 1) ? pw[0][b] >> 4 : pw[0][b]) & 0x000f000fu) | k6464;
         const uint32_t n23 = (((z & 1) ? pw[1][b] >> 4 : pw[1][b]) & 0x000f000fu) | k6464;
@@ -879,61 +881,179 @@ __device__ __forceinline__ void consume_pair_tiles(State<D>& st, const Tile<D, N
 }
 
 // A Q4-20B tile of a contiguous walk (aligned blocks of >= 16 tokens, zone
-// units of 32) at head_dim 64: its 16 K rows and its 16 V rows are each one
-// span of 16 * 40 bytes, together 80 chunks of 16 bytes.  Lane l takes chunk
-// l of K then V (lanes 0-39 the K chunks, 40-63 the first 24 V chunks) with
-// one 16-byte load, and bytes 384 + 4l of the V span with one 4-byte load:
-// five registers a tile, every byte loaded once.
+// units of 32): its 16 K rows and its 16 V rows are each one span of 16 * TS
+// bytes.  The K span and then the V span are taken as 16-byte chunks, chunk
+// 64 i + l by lane l with load i, while whole loads of 64 chunks fit (one at
+// head_dim 64, two at 128); the remaining bytes of the V span are 4 (8) per
+// lane: five (ten) registers a tile, every byte loaded once.
 template <int D>
 struct SpanTile {
-    static_assert(D == 64, "span tiles: head_dim 64");
     static constexpr int TS = q4_row_bytes(D);
-    static constexpr int KCH = TS;                // 16-byte chunks of a span
-    static constexpr int VTAIL = 16 * (64 - KCH);  // V bytes in the 16-byte loads
-    u32x4a c;
-    uint32_t w;
+    static constexpr int LOADS = 32 * TS / 1024;               // 16-byte loads per lane
+    static constexpr int TAILW = (32 * TS - 1024 * LOADS) / 256;  // tail words per lane
+    static constexpr int VTAIL = 1024 * LOADS - 16 * TS;       // V bytes in the 16-byte loads
+    u32x4a c[LOADS];
+    uint32_t w[TAILW];
 };
 
 template <int D>
 __device__ __forceinline__ void load_span(SpanTile<D>& t, const void* kb, const void* vb, long long base,
                                           int lane) {
-    constexpr int KCH = SpanTile<D>::KCH, VTAIL = SpanTile<D>::VTAIL;
-    const uint8_t* p = lane < KCH ? (const uint8_t*)kb + 16 * lane : (const uint8_t*)vb + 16 * (lane - KCH);
-    t.c = __builtin_nontemporal_load((const u32x4a*)(p + base));
-    t.w = __builtin_nontemporal_load((const uint32_t*)((const uint8_t*)vb + VTAIL + 4 * lane + base));
+    using T = SpanTile<D>;
+#pragma unroll
+    for (int i = 0; i < T::LOADS; i++) {
+        const int o = 1024 * i + 16 * lane;  // in the K span followed by the V span
+        const uint8_t* p = o < 16 * T::TS ? (const uint8_t*)kb + o : (const uint8_t*)vb + (o - 16 * T::TS);
+        t.c[i] = __builtin_nontemporal_load((const u32x4a*)(p + base));
+    }
+    const uint8_t* pw = (const uint8_t*)vb + T::VTAIL + 4 * T::TAILW * lane + base;
+    if constexpr (T::TAILW == 1) {
+        t.w[0] = __builtin_nontemporal_load((const uint32_t*)pw);
+    } else {
+        const u32x2a w = __builtin_nontemporal_load((const u32x2a*)pw);
+        t.w[0] = w[0];
+        t.w[1] = w[1];
+    }
 }
 
-// Operands of a span tile: the chunks go to one of the wavefront's two LDS
-// slots (rows at TS-byte strides, K then V), from which each lane reads the
-// words the tile layout gives it (Tile<D, Q4-20B>: K row j's nibble words, V
-// rows 4kq+r's header and nibbles) and the K headers of rows 4kq+r
-// (khr[g][r]).  The wavefront's LDS operations complete in order: a later
-// tile's writes to the slot come after these reads.
+// The wavefront's two LDS slots of a span tile: K rows and then V rows at
+// TS-byte strides.  The wavefront's LDS operations complete in order: a later
+// tile's writes to a slot come after the reads of the one before.
 template <int D>
-__device__ __forceinline__ void stage_span(const SpanTile<D>& sp, Tile<D, NYION_KV_Q4_20B>& t,
-                                           uint32_t (*khr)[4], int j, int kq, int slot = 0) {
-    constexpr int TS = SpanTile<D>::TS, DPL = D / 16;
-    // K at bytes 0 .. 16 TS - 1 of the slot, V after it
-    __shared__ u32x4 sm_span[4][2][2 * SpanTile<D>::KCH];
+__device__ __forceinline__ u32x4* span_slot(int slot) {
+    __shared__ u32x4 sm_span[4][2][2 * SpanTile<D>::TS];
+    return sm_span[threadIdx.x >> 6][slot];
+}
+
+template <int D>
+__device__ __forceinline__ void put_span(const SpanTile<D>& sp, u32x4* sb) {
+    using T = SpanTile<D>;
     const int lane = threadIdx.x & 63;
-    u32x4* sb = sm_span[threadIdx.x >> 6][slot];
-    sb[lane] = sp.c;                         // bytes 0 .. 1023: K, then V bytes 0 .. 383
-    ((uint32_t*)(sb + 64))[lane] = sp.w;     // V bytes 384 + 4 lane
+#pragma unroll
+    for (int i = 0; i < T::LOADS; i++) sb[64 * i + lane] = sp.c[i];
+    uint32_t* sw = (uint32_t*)(sb + 64 * T::LOADS) + T::TAILW * lane;  // the V span's tail
+    if constexpr (T::TAILW == 1)
+        sw[0] = sp.w[0];
+    else
+        *(u32x2*)sw = u32x2{sp.w[0], sp.w[1]};
+}
+
+// The words of a staged tile that the tile layout gives lane (j, kq): K row
+// j's nibble words; the K headers of rows 4kq+r (khr[g][r]); V rows 4kq+r's
+// header and nibbles.
+template <int D, bool NIBBLES, bool HEADERS>
+__device__ __forceinline__ void span_k(const u32x4* sb, Tile<D, NYION_KV_Q4_20B>& t, uint32_t (*khr)[4],
+                                       int j, int kq) {
+    constexpr int TS = SpanTile<D>::TS;
     const uint8_t* kr = (const uint8_t*)sb;
-    const uint8_t* vr = kr + 16 * TS;
 #pragma unroll
     for (int g = 0; g < D / 32; g++) {
-        t.kn[g] = *(const uint32_t*)(kr + TS * j + kQ4GroupBytes * g + 4 + 4 * kq);
+        if (NIBBLES) t.kn[g] = *(const uint32_t*)(kr + TS * j + kQ4GroupBytes * g + 4 + 4 * kq);
+        if (HEADERS) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) khr[g][r] = *(const uint32_t*)(kr + TS * (4 * kq + r) + kQ4GroupBytes * g);
+            for (int r = 0; r < 4; r++) khr[g][r] = *(const uint32_t*)(kr + TS * (4 * kq + r) + kQ4GroupBytes * g);
+        }
     }
+}
+
+template <int D>
+__device__ __forceinline__ void span_v(const u32x4* sb, Tile<D, NYION_KV_Q4_20B>& t, int j, int kq) {
+    constexpr int TS = SpanTile<D>::TS, DPL = D / 16;
+    const uint8_t* vr = (const uint8_t*)sb + 16 * TS;
     const int gv = (DPL * j) >> 5;                  // the group of the lane's V dims
     const int nv = 4 + (((DPL * j) & 31) >> 1);     // their first nibble byte in the group
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const uint8_t* row = vr + TS * (4 * kq + r) + kQ4GroupBytes * gv;
         t.vhdr[r] = *(const uint32_t*)row;
-        t.v[r] = *(const uint16_t*)(row + nv);  // head_dim 64: four dims, two bytes
+        if constexpr (D == 64)
+            t.v[r] = *(const uint16_t*)(row + nv);  // four dims, two bytes
+        else
+            t.v[r] = *(const uint32_t*)(row + nv);  // eight dims
+    }
+}
+
+template <int D>
+__device__ __forceinline__ void stage_span(const SpanTile<D>& sp, Tile<D, NYION_KV_Q4_20B>& t,
+                                           uint32_t (*khr)[4], int j, int kq, int slot = 0) {
+    u32x4* sb = span_slot<D>(slot);
+    put_span<D>(sp, sb);
+    span_k<D, true, true>(sb, t, khr, j, kq);
+    span_v<D>(sb, t, j, kq);
+}
+
+// consume_pair_tiles for two tiles in the LDS slots, at head_dim 128: each
+// operand is read from its slot where it is used (the fences keep the reads
+// there), and the P.V operands are built for two output dims at a time, so
+// that the pair's words are never held in registers together and the ring of
+// four tiles fits beside it.
+//
+// Bound: vector issue (about 420 VALU instructions a pair, 300 of them the
+// exact V terms) with the two wavefronts of a SIMD covering each other's LDS
+// and memory waits.  24 sequences of 200-16000 tokens, 32/8 heads: per-row
+// loads 110.3 us, span tiles one at a time with a ring of two 83.1 (three
+// and four, spilling: 88.2, 95.6), pairs and a ring of two 86.1, of four
+// 77.2; four dims at a time spill (88.2).  K headers exchanged through a
+// second slot instead of re-read per row: 79.3.  At head_dim 64 the pair fits
+// in registers, and reading it here ran 95.6 -> 101.4 us (64 sequences).
+template <int D, bool MASKED>
+__device__ __forceinline__ void consume_pair_staged(State<D>& st, const float* qv, uint32_t ma, uint32_t mb,
+                                                    int j, int kq, float scale_log2) {
+    constexpr int KVT = NYION_KV_Q4_20B;
+    constexpr int DPL = D / 16;
+    const u32x4 *sa = span_slot<D>(0), *sb = span_slot<D>(1);
+    auto scores = [&](const u32x4* slot) __attribute__((always_inline)) {
+        Tile<D, KVT> t;
+        floatx4 sg[D / 32];
+        uint32_t khr[D / 32][4];
+        span_k<D, true, false>(slot, t, khr, j, kq);
+        q4_tile_mfma<D>(t, qv, sg);
+        span_k<D, false, true>(slot, t, khr, j, kq);
+        return q4_tile_combine<D>(sg, qv, khr);
+    };
+    float sv[8], pr[8];
+    __builtin_amdgcn_s_setprio(1);
+    const floatx4 xa = scores(sa);
+    asm volatile("" ::: "memory");
+    const floatx4 xb = scores(sb);
+    if constexpr (!MASKED) {
+        const float x[8] = {xa[0], xa[1], xa[2], xa[3], xb[0], xb[1], xb[2], xb[3]};
+        softmax_step_raw<D, 8>(st, x, scale_log2 * 16777216.f, kq, pr);
+    } else {
+        tile_logits<KVT, true, false>(xa, scale_log2, ma, kq, nullptr, nullptr, sv);
+        tile_logits<KVT, true, false>(xb, scale_log2, mb, kq, nullptr, nullptr, sv + 4);
+        softmax_step<D, KVT, 8>(st, sv, kq, pr);
+    }
+    const halfx8 pa = {(_Float16)pr[0], (_Float16)pr[1], (_Float16)pr[2], (_Float16)pr[3],
+                       (_Float16)pr[4], (_Float16)pr[5], (_Float16)pr[6], (_Float16)pr[7]};
+    __builtin_amdgcn_s_setprio(0);
+    asm volatile("" ::: "memory");
+    Tile<D, KVT> ta, tb;
+    span_v<D>(sa, ta, j, kq);
+    span_v<D>(sb, tb, j, kq);
+    auto products = [&](auto z0) __attribute__((always_inline)) {
+        constexpr int Z0 = decltype(z0)::value, Z1 = Z0 + 2;
+        const Q4VOperands<D> oa = q4_v_operands<D, MASKED, Z0, Z1>(ta, ma, kq, st.k6464);
+        const Q4VOperands<D> ob = q4_v_operands<D, MASKED, Z0, Z1>(tb, mb, kq, st.k6464);
+        if (Z0 == 0)
+            st.acc_m = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                pa, __builtin_bit_cast(halfx8, u32x4{oa.mm[0], oa.mm[1], ob.mm[0], ob.mm[1]}), st.acc_m, 0, 0, 0);
+#pragma unroll
+        for (int z = Z0; z < Z1; z++) {
+            st.acc[z] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                pa, __builtin_bit_cast(halfx8, u32x4{oa.hi[z][0], oa.hi[z][1], ob.hi[z][0], ob.hi[z][1]}),
+                st.acc[z], 0, 0, 0);
+            st.acc[z] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                pa, __builtin_bit_cast(halfx8, u32x4{oa.lo[z][0], oa.lo[z][1], ob.lo[z][0], ob.lo[z][1]}),
+                st.acc[z], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    products(std::integral_constant<int, 0>{});
+    products(std::integral_constant<int, 2>{});
+    if constexpr (DPL > 4) {
+        products(std::integral_constant<int, 4>{});
+        products(std::integral_constant<int, 6>{});
     }
 }
 
@@ -1113,22 +1233,26 @@ __device__ __forceinline__ uint32_t global_offsets(const DecodeArgs& a, const Ex
     return mask;
 }
 
-// Contiguous walks load Q4-20B tiles as spans at head_dim 64; head_dim 128
-// keeps per-row loads (twice the bytes per load; its span tiles and staged
-// operands exceed the register budget).
+// Contiguous walks load Q4-20B tiles as spans: the 13 scattered 4-byte loads
+// of a per-row tile become three wide ones (at head_dim 128, one sequence of
+// 4096 tokens 13.9 -> 13.4 us, 8 of 300-3000 24.2 -> 18.3, 64 of 512-16000 on
+// 8/2 heads 76.4 -> 53.8, 8 windows of 4096 28.5 -> 23.8).
 template <int D, int KVT>
 constexpr bool span_tiles() {
-    return KVT == NYION_KV_Q4_20B && D == 64;
+    return KVT == NYION_KV_Q4_20B;
 }
 
 // Tiles whose loads a wavefront keeps in flight: the one being consumed and
-// NB - 1 ahead.  A Q4-20B span tile (head_dim 64) is 1280 bytes, a sixth of
-// an f32 tile, so it takes a ring of four.  Gathered tiles (position lists,
-// strided globals) keep two: their walks are short, and the extra tiles
-// loaded past a walk's end cost more than the deeper ring gains.
-template <int D, int KVT, bool SPAN>
+// NB - 1 ahead.  A Q4-20B span tile is 1280 bytes at head_dim 64, a sixth of
+// an f32 tile, so it takes a ring of four; at head_dim 128 too, except for
+// tracked walks, whose scores leave no registers for it (4 sequences of
+// 3000-9000 tokens: per-row loads 33.8 us, a ring of two 28.9, of four 39.5).
+// Gathered tiles (position lists, strided globals) keep two: their walks are
+// short, and the extra tiles loaded past a walk's end cost more than the
+// deeper ring gains.
+template <int D, int KVT, bool SPAN, bool TRACK>
 constexpr int tile_ring() {
-    return SPAN ? 4 : 2;
+    return SPAN && !(TRACK && D == 128) ? 4 : 2;
 }
 
 // Walk `n` tiles with the next NB - 1 tiles' loads in flight during each MFMA
@@ -1146,7 +1270,7 @@ __device__ __forceinline__ void walk_tiles(State<D>& st, const DecodeArgs& a, co
     // untracked span tiles go in pairs (the tracked form's score positions
     // leave no registers for the second staged tile)
     constexpr bool PAIRS = SPAN && !TRACK;
-    constexpr int NB = tile_ring<D, KVT, SPAN>();
+    constexpr int NB = tile_ring<D, KVT, SPAN, TRACK>();
     static_assert(!PAIRS || NB % 2 == 0, "pairs take slots 2i, 2i+1");
     using RingTile = typename std::conditional<SPAN, SpanTile<D>, Tile<D, KVT>>::type;
     RingTile t[NB];
@@ -1171,6 +1295,15 @@ __device__ __forceinline__ void walk_tiles(State<D>& st, const DecodeArgs& a, co
         // before that step's load refills slot k-1
         auto eat_pair = [&](const RingTile& x, const RingTile& y, uint32_t ma, uint32_t mb, const int* pa,
                             const int* pb) {
+            if constexpr (D == 128) {
+                put_span<D>(x, span_slot<D>(0));
+                put_span<D>(y, span_slot<D>(1));
+                if ((ma & mb) == 0xffffu)
+                    consume_pair_staged<D, false>(st, qv, ma, mb, j, kq, a.scale_log2);
+                else
+                    consume_pair_staged<D, true>(st, qv, ma, mb, j, kq, a.scale_log2);
+                return;
+            }
             Tile<D, KVT> ya, yb;
             uint32_t khra[D / 32][4], khrb[D / 32][4];
             stage_span<D>(x, ya, khra, j, kq, 0);
