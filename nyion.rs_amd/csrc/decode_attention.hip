@@ -5,12 +5,14 @@
 // (swamp-engine/src/ops.rs:170-278) and ops::attention_sparse (ops.rs:85-168);
 // the header states the position sets.
 //
-// Work decomposition (stream-K).  A segment is one (sequence, kv head, group
-// of up to 16 q heads); its attended positions form a list of 16-token tiles.
-// The segments' tile lists are laid end to end and a grid sized to the
+// Work decomposition.  A segment is one (sequence, kv head, group of up to 16
+// q heads); its attended positions form a list of 16-token tiles.  Stream-K:
+// the segments' tile lists are laid end to end and a grid sized to the
 // resident capacity of the chip cuts that list into equal ranges, one per
 // 256-thread workgroup, whatever the spread of context lengths.  A workgroup
 // walks its range segment by segment; its four wavefronts split each piece.
+// Launches of few segments cut each segment by itself instead, one piece per
+// workgroup (DecodePart).
 // All q heads of a GQA group are processed together, so each K/V byte is read
 // from HBM once.
 //
@@ -75,6 +77,15 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 enum DecodeMode { MODE_FULL = 0, MODE_WINDOW = 1, MODE_LIST = 2 };
 
+// How a launch's workgroups take the segments' tiles: ranges of the segments'
+// tile lists laid end to end; the host's equal number of pieces per segment;
+// pieces in proportion to the lengths (ragged_piece).  One kernel each: with
+// all in one the walk's scalar state spilled, and without the stream-K form
+// the direct ones need 30-40 vector registers less and spill nothing (one
+// tracked sequence of 4096 tokens 15.4 -> 14.3 us, 8 windows of 4096 15.4 ->
+// 14.5, one binary16 sequence of 4096 at head_dim 128 13.6 -> 12.6).
+enum DecodePart { PART_STREAM = 0, PART_DIRECT = 1, PART_RAGGED = 2 };
+
 struct DecodeArgs {
     const float* q;  // [B][Hq][D]
     const void* k;
@@ -111,6 +122,8 @@ struct DecodeArgs {
     unsigned* status;  // the device's range-status word (binary16 q overflow)
     int direct;        // > 0: direct partition, pieces per segment (else stream-K)
     int seg_tiles;     // direct: host bound on the tiles of one segment
+    int ragged_min;    // > 0: direct, pieces in proportion to the lengths
+                       // (ragged_pieces), this many tiles or more each
     int spec_len;      // window mode: the host's max_ctx, whose window start a
                        // walk's block-table loads may assume before the
                        // length arrives (0: none)
@@ -184,6 +197,62 @@ __device__ __forceinline__ Extent extent_of(const DecodeArgs& a, int2 v) {
 }
 
 // Extent of sequence b as seen by one thread (no uniformity assumed).
+// Inclusive prefix sum over the wavefront (every lane active), on DPP row
+// shifts and row broadcasts.
+__device__ __forceinline__ int wave_scan(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
+    return x;
+}
+
+// Direct partition of a full-context batch in proportion to the lengths: the
+// workgroup's piece.  The host knows only the longest context, and with its
+// equal cut a launch lasts as long as the longest sequence's pieces while the
+// workgroups of the others idle (8 binary16 sequences of 300-3000 tokens, 32/8
+// heads of 128: 23.7 -> 19.7 us; of 4000-16000 77.5 -> 62.5; f32 39.0 -> 30.9;
+// equal lengths of 3000: 25.7 -> 25.4).  Every segment is cut into ceil(tiles / c) pieces (at
+// least one), with one c for all, the smallest of a few candidates at which
+// the batch's pieces number at most the grid: from the even share of all
+// tiles (exact when the lengths are equal: the host's own cut) towards the
+// bound that always fits.  Each wavefront computes it for itself, lane l
+// holding sequence l (at most 64), without barriers.
+struct RaggedPiece {
+    int b, u, piece, pieces, first;  // first: the workgroup of the segment's piece 0
+    int2 v;                          // the sequence's (length, q position)
+};
+
+template <bool ALIGNED>
+__device__ __forceinline__ RaggedPiece ragged_piece(const DecodeArgs& a, int U, int g, int lane) {
+    const bool in = lane < a.batch;
+    const int2 v = seq_values(a, in ? lane : 0);
+    const int t = in ? max(1, extent_of<ALIGNED>(a, v).tiles) : 0;
+    auto total = [](int scan) { return __builtin_amdgcn_readlane(scan, 63); };
+    const int T = total(wave_scan(t)) * U, segs = a.batch * U, grid = a.decode_grid;
+    const int fits = (T + grid - segs - 1) / (grid - segs);  // sum of ceil(t/c) <= T/c + segs <= grid
+    int c = max(a.ragged_min, (T + grid - 1) / grid), pc = 0, incl = 0;
+    for (int i = 0;; i++) {
+        pc = (t + c - 1) / c;
+        incl = wave_scan(pc);
+        if (i == 3 || total(incl) * U <= grid) break;
+        c = i == 2 ? fits : (c + fits) / 2 + 1;
+    }
+    RaggedPiece r;
+    r.b = __popcll(__ballot(in && incl * U <= g));
+    if (r.b < a.batch) {
+        r.pieces = __builtin_amdgcn_readlane(pc, r.b);
+        const int g0 = U * (__builtin_amdgcn_readlane(incl, r.b) - r.pieces);
+        r.u = (g - g0) / r.pieces;
+        r.first = g0 + r.u * r.pieces;
+        r.piece = g - r.first;
+        r.v = int2{__builtin_amdgcn_readlane(v.x, r.b), __builtin_amdgcn_readlane(v.y, r.b)};
+    }
+    return r;
+}
+
 template <bool ALIGNED>
 __device__ __forceinline__ Extent lane_extent(const DecodeArgs& a, int b) {
     return extent_of<ALIGNED>(a, seq_values(a, b));
@@ -1661,7 +1730,7 @@ __global__ __launch_bounds__(256) void importance_kernel(DecodeArgs a, double* i
     importance_body(a, imp, imp_stride, blockIdx.x, blockIdx.y, gridDim.y, sml, part);
 }
 
-template <int D, int KVT, bool ALIGNED, bool TRACK, bool ZONE = false>
+template <int D, int KVT, bool ALIGNED, bool TRACK, bool ZONE, int PART>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(decode_waves_per_eu<D, KVT>())))
 void decode_kernel(DecodeArgs a) {
@@ -1708,12 +1777,14 @@ void decode_kernel(DecodeArgs a) {
     // segment's tiles, one iteration, no per-workgroup prefix sums; with full
     // context a tile's positions do not depend on the length, so this
     // wavefront's block-table entries are requested before the length
-    // arrives.  Stream-K (otherwise): the segments' tile lists laid end to
-    // end and cut into equal ranges, one per workgroup, possibly spanning
-    // several segments.
-    const bool direct = a.direct > 0;
+    // arrives.  Ragged: the same, but the segment and piece follow from the
+    // lengths; the entries are requested for the host's cut all the same and
+    // kept where the two agree (equal lengths).  Stream-K (otherwise): the
+    // segments' tile lists laid end to end and cut into equal ranges, one per
+    // workgroup, possibly spanning several segments.
+    constexpr bool direct = PART != PART_STREAM, RAGGED = PART == PART_RAGGED;
     int g1 = 0, c = 1, pos = 0, b = 0;
-    if (!direct) {
+    if constexpr (!direct) {
         // tiles of one segment of each sequence, prefix-summed into LDS
         int carry = 0;
         if (threadIdx.x == 0) sm_pref[0] = 0;
@@ -1767,23 +1838,23 @@ void decode_kernel(DecodeArgs a) {
         bool whole, pref = false;
         int tbl_pref = -1;
         Extent e;
-        if (direct) {
+        if constexpr (direct) {
             const int P = a.direct;
             const int s = (int)blockIdx.x / P;
-            const int piece = (int)blockIdx.x - s * P;
+            int piece = (int)blockIdx.x - s * P;
             b = s / U;
             u = s - b * U;
-            const int cd = (a.seg_tiles + P - 1) / P;
-            const int t0 = piece * cd;
-            const int wa0 = t0 + (wave * cd) / 4, wb0 = t0 + ((wave + 1) * cd) / 4;
-            pref = ALIGNED && a.mode == MODE_FULL && a.tables && wb0 > wa0;
+            int cd = (a.seg_tiles + P - 1) / P;
+            int t0 = piece * cd;
+            int wa0 = t0 + (wave * cd) / 4, wb0 = t0 + ((wave + 1) * cd) / 4;
+            pref = ALIGNED && (RAGGED || a.mode == MODE_FULL) && a.tables && wb0 > wa0;
             // untracked 4-bit span walks of paged windows: the walk of a
             // sequence at the host's max_ctx (q at its end) starts at block
             // position pref_base; its entries are requested with the length,
             // kept if the extent confirms that start
             constexpr bool kSpec = tile_table<KVT, ZONE>() && span_tiles<D, KVT>() && !TRACK;
             int pref_base = 0;
-            if (kSpec && ALIGNED && a.mode == MODE_WINDOW && a.spec_len > 0 && a.tables && wb0 > wa0) {
+            if (kSpec && !RAGGED && ALIGNED && a.mode == MODE_WINDOW && a.spec_len > 0 && a.tables && wb0 > wa0) {
                 const int ve = a.spec_len - 1;
                 pref_base = (ve > a.window ? ve - a.window + 1 : 0) & ~15;
                 pref = true;
@@ -1791,12 +1862,34 @@ void decode_kernel(DecodeArgs a) {
             if (pref)
                 tbl_pref = run_table_entry<tile_table<KVT, ZONE>()>(
                     a, a.tables + (long long)b * a.table_stride, pref_base, wa0, min(64, wb0 - wa0), lane);
-            const int len = a.ctx_lens ? sload(a.ctx_lens + b) : a.uniform_len;
-            const int qp = a.q_pos ? sload(a.q_pos + b) : len - 1;
-            e = extent_of<ALIGNED>(a, int2{len, qp});
+            whole = P == 1;
+            pieces = P;
+            slot = (int)blockIdx.x;
+            slot0 = (long long)s * P;
+            if constexpr (RAGGED) {
+                const RaggedPiece r = ragged_piece<ALIGNED>(a, U, (int)blockIdx.x, lane);
+                if (r.b >= a.batch) return;  // more workgroups than pieces
+                e = extent_of<ALIGNED>(a, r.v);
+                cd = (e.tiles + r.pieces - 1) / r.pieces;
+                t0 = r.piece * cd;
+                const int wa1 = t0 + (wave * cd) / 4, wb1 = t0 + ((wave + 1) * cd) / 4;
+                // the entries loaded ahead are those of the host's cut
+                pref = pref && r.b == b && wa1 == wa0 && wb1 <= wb0;
+                b = r.b;
+                u = r.u;
+                wa0 = wa1;
+                wb0 = wb1;
+                whole = r.pieces == 1;
+                pieces = r.pieces;
+                slot0 = r.first;
+            } else {
+                const int len = a.ctx_lens ? sload(a.ctx_lens + b) : a.uniform_len;
+                const int qp = a.q_pos ? sload(a.q_pos + b) : len - 1;
+                e = extent_of<ALIGNED>(a, int2{len, qp});
+            }
             wa = min(wa0, e.tiles);
             wb = min(wb0, e.tiles);
-            if (KVT == NYION_KV_Q4_20B && ALIGNED && e.n_glob > 0 && e.main_tiles > t0 &&
+            if (KVT == NYION_KV_Q4_20B && ALIGNED && !RAGGED && e.n_glob > 0 && e.main_tiles > t0 &&
                 e.main_tiles < t0 + cd) {
                 // no wavefront walks both sides of the boundary between the
                 // contiguous tiles and the globals (two serial chains of round
@@ -1815,10 +1908,6 @@ void decode_kernel(DecodeArgs a) {
             // (the entries cover tiles wa0 .. wb0 - 1: a walk start moved or
             // an end moved past wb0 by the re-cut above loads its own)
             if (kSpec && pref && ((e.lo & ~15) != pref_base || wa != wa0 || wb > wb0)) pref = false;
-            whole = P == 1;
-            pieces = P;
-            slot = (int)blockIdx.x;
-            slot0 = (long long)s * P;
         } else {
             while (U * sload(&sm_pref[b + 1]) <= pos) b++;
             const int pb = sload(&sm_pref[b]);
@@ -2180,7 +2269,7 @@ static int resident_capacity() {
         cache,
         [] {
             int per_cu = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_kernel<D, KVT, AL, TR, ZN>,
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_kernel<D, KVT, AL, TR, ZN, PART_STREAM>,
                                                              256, 0) != hipSuccess) {
                 (void)hipGetLastError();
                 return 0;
@@ -2269,6 +2358,8 @@ static void launch_dk(const DecodePlan& pl, hipStream_t stream) {
                 a.direct = (int)P;
                 a.seg_tiles = seg_tiles;
                 grid = (int)(P * segs);
+                if (a.mode == MODE_FULL && nb > 1 && P > 1 && a.ctx_lens)
+                    a.ragged_min = std::min<int>(wgd, (int)((seg_tiles + P - 1) / P));
             }
         }
         a.decode_grid = grid;
@@ -2281,8 +2372,12 @@ static void launch_dk(const DecodePlan& pl, hipStream_t stream) {
             a.imp_batch = pl.batch;
             launch += (long long)a.imp_nx * a.imp_ny;
         }
-        hipLaunchKernelGGL((decode_kernel<D, KVT, AL, TR, ZN>), dim3((unsigned)launch), dim3(256), 0,
-                           stream, a);
+        auto kernel = decode_kernel<D, KVT, AL, TR, ZN, PART_STREAM>;
+        if constexpr (AL) {
+            if (a.ragged_min > 0) kernel = decode_kernel<D, KVT, AL, TR, ZN, PART_RAGGED>;
+            else if (a.direct > 0) kernel = decode_kernel<D, KVT, AL, TR, ZN, PART_DIRECT>;
+        }
+        hipLaunchKernelGGL(kernel, dim3((unsigned)launch), dim3(256), 0, stream, a);
     }
 }
 
