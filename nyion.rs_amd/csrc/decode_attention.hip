@@ -2290,6 +2290,18 @@ static int wg_tiles_for(long long total_tiles) {
 // segments the stream-K prologue (lengths, prefix sums, a search) is a
 // dependent round trip and two barriers that the direct form skips.
 constexpr int kDirectMaxSegments = 64;
+// Full-context batches (at most 64 sequences, one per lane of ragged_piece)
+// take the ragged form up to more segments while the K and V that their bound
+// allows stay below kRaggedMaxBytes: it saves the stream-K prologue and the
+// merges of ranges that span segments, about 7 us, against a cut up to
+// grid / (grid - segments) from even.  Measured (us, stream-K / ragged): 24
+// 4-bit sequences of 300-3000 tokens (32/4 heads of 64, 23 MB) 20.2 / 15.0, 64
+// of them (61 MB) 29.3 / 20.9, 12 binary16 ones (32/8 heads of 128, 148 MB)
+// 29.8 / 25.5, 32 f32 ones (32/4 of 64, 192 MB) 33.2 / 29.7, and beyond: 48
+// (8/2 of 128, 289 MB) 51.5 / 59.0, 24 binary16 ones (296 MB) 43.2 / 45.4, 24
+// 4-bit ones of 200-16000 (491 MB) 76.9 / 91.3.
+constexpr int kRaggedMaxSegments = 256;
+constexpr long long kRaggedMaxBytes = 200LL << 20;
 // Direct partition of small tiles (4-bit rows, binary16 at head_dim 64): the
 // tiles per workgroup double while a workgroup's K+V bytes stay within
 // kDirectWgBytes and the launch keeps kDirectMinGrid workgroups.  Such a
@@ -2305,12 +2317,16 @@ constexpr long long kDirectWgBytes = 96 << 10;
 constexpr long long kDirectMinGrid = 128;
 constexpr int kDirectMinPieceTiles = 16;
 
+// K and V bytes of one tile.
+template <int D, int KVT>
+constexpr long long tile_bytes() {
+    return 32LL * (KVT == NYION_KV_Q4_20B ? q4_row_bytes(D) : KVT == NYION_KV_F16 ? 2 * D : 4 * D);
+}
+
 template <int D, int KVT>
 static int direct_wg_tiles(int wg, int seg_tiles, long long segs) {
     if (g_wg_tiles_override.load(std::memory_order_relaxed) > 0) return wg;
-    constexpr long long tile_bytes =
-        32LL * (KVT == NYION_KV_Q4_20B ? q4_row_bytes(D) : KVT == NYION_KV_F16 ? 2 * D : 4 * D);
-    while (2 * wg * tile_bytes <= kDirectWgBytes && 2 * wg <= seg_tiles &&
+    while (2 * wg * tile_bytes<D, KVT>() <= kDirectWgBytes && 2 * wg <= seg_tiles &&
            (seg_tiles + 2LL * wg - 1) / (2LL * wg) * segs >= kDirectMinGrid)
         wg *= 2;
     return wg;
@@ -2340,10 +2356,13 @@ static void launch_dk(const DecodePlan& pl, hipStream_t stream) {
         if (grid > pl.grid_bound) grid = pl.grid_bound;
         if (pl.ws_bytes == 0 || (nb == 1 && grid <= units)) grid = units;  // whole segments
         const long long segs = (long long)nb * units;
-        if (AL && a.mode != MODE_LIST && segs <= kDirectMaxSegments) {
+        const int seg_tiles = a.mode == MODE_FULL ? (a.max_len + 15) / 16 : pl.tiles_max;
+        const bool ragged = a.mode == MODE_FULL && nb > 1 && nb <= 64 && a.ctx_lens && pl.ws_bytes != 0;
+        if (AL && a.mode != MODE_LIST &&
+            (segs <= kDirectMaxSegments ||
+             (ragged && segs <= kRaggedMaxSegments && segs * seg_tiles * tile_bytes<D, KVT>() <= kRaggedMaxBytes))) {
             // pieces per segment from the tiles per workgroup, within the
             // partial slots the workspace holds (one per workgroup)
-            const int seg_tiles = a.mode == MODE_FULL ? (a.max_len + 15) / 16 : pl.tiles_max;
             const int wgd = direct_wg_tiles<D, KVT>(wg, seg_tiles, segs);
             long long P = pl.ws_bytes == 0 ? 1 : (seg_tiles + wgd - 1) / wgd;
             if (pl.ws_bytes != 0 && wgd > wg) {
@@ -2354,11 +2373,15 @@ static void launch_dk(const DecodePlan& pl, hipStream_t stream) {
             }
             const long long limit = std::min<long long>(cap, pl.grid_bound);
             if (P * segs > limit) P = std::max<long long>(1, limit / segs);
-            if (P > 1 || pl.ws_bytes == 0 || nb == 1) {
+            // one piece: where a workgroup is meant to take a whole segment (a
+            // batch of short contexts: 8 f32 sequences of 128 tokens 13.7 -> 6.1
+            // us, 32 binary16 ones of 10-100 at head_dim 128 21.2 -> 6.4), not
+            // where the resident grid holds no more
+            if (P > 1 || pl.ws_bytes == 0 || nb == 1 || seg_tiles <= wgd) {
                 a.direct = (int)P;
                 a.seg_tiles = seg_tiles;
                 grid = (int)(P * segs);
-                if (a.mode == MODE_FULL && nb > 1 && P > 1 && a.ctx_lens)
+                if (ragged && P > 1)
                     a.ragged_min = std::min<int>(wgd, (int)((seg_tiles + P - 1) / P));
             }
         }

@@ -1,10 +1,11 @@
 """Full-context decode batches whose pieces follow the lengths (gpu).
 
-With at most 64 segments every segment is cut into pieces in proportion to its
-tiles.  The batches: all lengths equal (the cut is the host's), one long
-sequence among short, empty and one-token ones, 64 sequences (a whole
-wavefront of lengths), fewer pieces than workgroups, and partition sizes from
-one tile per wavefront to whole segments.  Tolerance as for every attention
+In a batch of at most 64 sequences and 256 segments every segment is cut into
+pieces in proportion to its tiles, or is one piece.  The batches: all lengths
+equal (the cut is the host's), one long sequence among short and one-token
+ones, 64 sequences (a whole wavefront of lengths), fewer pieces than
+workgroups, the limits of the rule and one segment more, and partition sizes
+from one tile per wavefront to whole segments.  Tolerance as for every attention
 output (test_decode_gpu).
 """
 import numpy as np
@@ -24,6 +25,10 @@ BATCHES = {
     "two": ([31, 2049], 8, 2),
     "64 sequences": (list(range(1, 630, 10)) + [1500], 4, 1),
     "short": ([1, 2, 3, 4, 5, 6, 7, 8], 16, 8),
+    "many": ([30 + 37 * i for i in range(24)], 16, 8),
+    "many short": (list(range(1, 121, 3)), 8, 4),
+    "256 segments": ([5 * i + 1 for i in range(64)], 4, 4),
+    "257 segments": ([300 - i for i in range(257)], 1, 1),
 }
 KINDS = [(oracle.KV_F32, 64), (oracle.KV_F16, 64), (oracle.KV_Q4, 64), (oracle.KV_F32, 128),
          (oracle.KV_F16, 128), (oracle.KV_Q4, 128)]
