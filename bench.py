@@ -819,8 +819,7 @@ def bench_c5(nh, torch, steps, warmup, seed=0):
         nh.prefill_bf16(q, k, v, out, Hq, Hkv, D, k_pool=kp, v_pool=vp, block_table=tab,
                         block_tokens=bt)
 
-    # the same chunk written into Q4-20B pools (the quantising write is its own
-    # launch after the attention kernel)
+    # the same chunk written into Q4-20B pools (quantised by the kernel itself)
     rbq = 4 * D // 32 * 5
     kq = torch.empty((nblk, Hkv, bt, rbq), dtype=torch.uint8, device="cuda")
     vq = torch.empty_like(kq)
