@@ -576,7 +576,8 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
         }
     };
     // the group's blocks in order: those of sum kg, then (KS = 1) of the next;
-    // nb past the last
+    // past the last nb, which may be b + kSumWays as well: a sum's end is told
+    // by b alone
     auto next_of = [&](int b) __attribute__((always_inline)) {
         if (b + kSumWays < nb) return b + kSumWays;
         const int k = b % kSumWays + 1;
@@ -643,7 +644,7 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
                 }
             }
         }
-        if (KS == 1 && b1 != b + kSumWays) {  // a sum is done (uniform)
+        if (KS == 1 && b + kSumWays >= nb) {  // a sum is done (uniform)
 #pragma unroll
             for (int i = 0; i < RT; i++)
 #pragma unroll

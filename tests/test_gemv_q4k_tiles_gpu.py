@@ -94,3 +94,34 @@ def test_q4k_input_extremes(gpu, n_cols, batch):
     assert np.isnan(again[0]).all() and np.isnan(again[batch - 1]).all()
     for b in range(1, batch - 1):
         assert np.array_equal(again[b], got[b].astype(np.float32)), b
+
+
+# (rows, inputs) for which the launch takes, on 256 CUs, the 32x16 and 64x16
+# tiles with their blocks in four K groups, and the 64x16, 128x32, 256x32 and
+# 384x32 tiles with one; remainders in both
+TILES = [(100, 33), (1500, 129), (5633, 33), (5633, 129), (4097, 260), (4097, 509)]
+
+
+@pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5, 6, 7, 8, 11, 43])
+@pytest.mark.parametrize("n_rows,batch", TILES)
+def test_q4k_every_tile(gpu, n_rows, batch, blocks):
+    """Every tile over row lengths of every remainder by the four sums, each sum
+    of none, one or several blocks: all outputs equal those of calls with eight
+    inputs (another kernel), and a sample of rows the float64 product."""
+    n_cols = 256 * blocks
+    w = W.q4k_random_weights(n_rows, n_cols, seed=blocks)
+    x = np.random.default_rng(batch).standard_normal((batch, n_cols)).astype(np.float32)
+    dw, dx = dev(w), dev(x)
+    out = torch.full((batch, n_rows), float("nan"), device="cuda")
+    few = torch.full((batch, n_rows), float("nan"), device="cuda")
+    gpu.gemv_q4k_batched(dw, dx, out, n_rows, n_cols)
+    for b in range(0, batch, 8):
+        gpu.gemv_q4k_batched(dw, dx[b:b + 8], few[b:b + 8], n_rows, n_cols)
+    torch.cuda.synchronize()
+    assert torch.equal(out, few)
+    rows = np.unique(np.linspace(0, n_rows - 1, 50).astype(int))
+    deq = W.q4k_dequant_np(w[rows], len(rows), n_cols).astype(np.float64).reshape(len(rows), n_cols)
+    ref = x.astype(np.float64) @ deq.T
+    bound = 8 * 2.0**-23 * (np.abs(x).astype(np.float64) @ np.abs(deq).T)
+    got = out[:, torch.from_numpy(rows).cuda()].cpu().numpy()
+    assert np.all(np.abs(got - ref) <= bound), np.max(np.abs(got - ref) / bound)
