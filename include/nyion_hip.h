@@ -581,10 +581,11 @@ int nyion_q4_quantize(const float* in, int64_t n_rows, int head_dim, uint8_t* ou
  * (swamp-kernels/src/fused_gemv_q4k.rs:59-99, 903-927), the Q4_K arm of
  * forward_linear (swamp-engine/src/linear.rs:99-189), with the f32
  * semantics of its scalar path (395-448).  Multiplied on binary16 matrix
- * cores: a block's integers exactly, x to within 2^-23 of each value (split
- * into two terms, scaled per 256 values), f32 sums.  n_cols a positive
- * multiple of 256; W and x 16-byte aligned.  out is written, not
- * accumulated. */
+ * cores: a block's integers exactly, x split into two terms to within 2^-23
+ * of each value or 2^-45 of the largest of its block's 256, whichever is more,
+ * f32 sums.  An infinity or NaN in x makes every output of that input NaN.
+ * n_cols a positive multiple of 256; W and x 16-byte aligned.  out is written,
+ * not accumulated. */
 int nyion_gemv_q4k(const uint8_t* d_w, const float* d_x, float* d_out, int n_rows, int n_cols,
                    nyion_stream_t stream);
 

@@ -17,16 +17,17 @@
 //    as small as the result: without it the error was 1.5 times larger);
 //  * each input's 256 values of a block are scaled by the power of two that
 //    brings their largest magnitude into [2^14, 2^15) and split into two
-//    binary16 terms, x = hi + lo to within 2^-23 of x (values below 2^-28 of
-//    the block's largest lose more of their own bits, never more than
-//    2^-39 of the largest); hi and lo have an accumulator each (lo added to
-//    hi's doubled the error).
+//    binary16 terms, x = hi + lo 2^-11, which hold it to within 2^-23 of x or
+//    2^-50 of the block's largest, whichever is more (2^-45 for the sums of x
+//    per sub-block, which are split likewise); hi and lo have an accumulator
+//    each (lo added to hi's doubled the error).
 // A block's value for one (row, input) is a chain of eight K steps, and an
 // output is the sum of kSumWays sums of its blocks' values, whichever kernel,
 // tile or wavefront computed them: single, multi-matrix and batched calls
-// give the same bits.  Against float64 the outputs are off by 1.5e-7 of their
-// norm (2048 to 4096 columns; f32 FMAs in runs of 16, as this file's products
-// were before, 1.7e-7 to 2.3e-7).
+// give the same bits.  Against float64 the outputs are off by 1.6e-7 to 1.7e-7
+// of their norm for N(0, 1) inputs (256 to 14336 columns; f32 FMAs in runs of
+// 16 were 1.8e-7 to 2.1e-7), and as much beside a value 2^24 times the others
+// under zero scales.
 //
 // Two kernels.  gemv_split_kernel (up to eight inputs): the wavefronts of a
 // workgroup take the blocks of 16 rows among them, each converting the inputs
@@ -71,6 +72,10 @@ __device__ __forceinline__ uint32_t half1024_reg() {
     return k;
 }
 
+// What the low terms of x count: they are kept 2^11 times larger, so that
+// they are normal binary16 numbers wherever the high terms are.
+constexpr float kLowTerm = 1.f / 2048;
+
 // ---------------------------------------------------------------------------
 // Weights.  Lane (n, g) of a wavefront (n = lane & 15 the row, g = lane >> 4)
 // holds 64 weights of its row's block, eight for each K step s = 0..7, as the
@@ -87,10 +92,11 @@ struct Q4k {
         u32x4 hdr, qa, qb;
     };
     // Scales of the two sub-blocks for the low nibbles' and the high nibbles'
-    // weights, scales and mins as operands of the sums of x, d and dmin.
+    // weights, scales and mins as operands of the sums of x (the mins also for
+    // their low terms), d and dmin.
     struct Scales {
         halfx2 s_lo, s_hi, c_hi;
-        uint32_t scales, mins;
+        uint32_t scales, mins, mins_low;
         float d, dmin;
     };
     __device__ static int x_offset(int s, int g) { return 64 * g + 4 * s; }
@@ -118,6 +124,7 @@ struct Q4k {
         c.c_hi = splat2(s.y) * splat2((_Float16)(-72.0 / 16384));
         c.scales = as_word(s * splat2((_Float16)(1.0 / 64)));
         c.mins = as_word(m);
+        c.mins_low = as_word(m * splat2((_Float16)kLowTerm));
         c.d = f16_bits_to_f32(r.hdr.x) * 16384.f;
         c.dmin = f16_bits_to_f32(r.hdr.x >> 16) * 32.f;
     }
@@ -178,24 +185,25 @@ __device__ __forceinline__ XShare load_x(const float* xb, int s, int g) {
 // The two binary16 terms of the share (operand words of step s, group g),
 // the block's 1 / scale, and, in the lanes with s = 0, the two terms of the
 // sums of x over sub-blocks 2g and 2g+1 (times 2^-5: the sum of 32 values
-// stays in range).  Whether x is finite does not matter here: an infinity or
-// NaN makes every output of its input that the reference's order of
-// operations makes NaN a NaN.
+// stays in range).  An infinity leaves a NaN in lo, so that it makes every
+// output of its input NaN, as a NaN does.
 struct XTerms {
     u32x4 hi, lo;
     uint32_t sum_hi, sum_lo;
     float inv;
 };
 
-// a and b as two binary16 terms each: the first holds the upper 11 bits,
-// rounded by integer operations on the f32 words (a third of the cycles of
-// converting back: v_fma_mix and the conversions issue at a quarter and half
-// the rate of and, add and subtract).
+// a and b as two binary16 terms each, a = hi + lo * kLowTerm.  The high term
+// is converted back to be subtracted, so that the low one also holds what a
+// denormal high term leaves (kept out of v_fma_mix, which issues at a quarter
+// of the rate of a subtraction).
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
-    const float ha = __uint_as_float((__float_as_uint(a) + 0x1000u) & 0xffffe000u);
-    const float hb = __uint_as_float((__float_as_uint(b) + 0x1000u) & 0xffffe000u);
-    hi = as_word(halfx2{(_Float16)ha, (_Float16)hb});
-    lo = as_word(halfx2{(_Float16)(a - ha), (_Float16)(b - hb)});
+    const halfx2 h = {(_Float16)a, (_Float16)b};
+    float ha = (float)h.x, hb = (float)h.y;
+    asm("" : "+v"(ha));
+    asm("" : "+v"(hb));
+    hi = as_word(h);
+    lo = as_word(halfx2{(_Float16)((a - ha) * (1.f / kLowTerm)), (_Float16)((b - hb) * (1.f / kLowTerm))});
 }
 
 __device__ __forceinline__ XTerms split_x(const XShare& x) {
@@ -229,11 +237,12 @@ __device__ __forceinline__ XTerms split_x(const XShare& x) {
     return t;
 }
 
-// x + the value of x 32 lanes on, in the lower half of the wavefront.
-__device__ __forceinline__ float add_other_half(float x) {
+// x + kLowTerm times the value of x 32 lanes on, in the lower half of the
+// wavefront.
+__device__ __forceinline__ float add_low_rows(float x) {
     const u32x2 r = __builtin_bit_cast(
         u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-    return __uint_as_float(r.x) + __uint_as_float(r.y);
+    return __builtin_fmaf(__uint_as_float(r.y), kLowTerm, __uint_as_float(r.x));
 }
 
 // An output is the sum of kSumWays sums, in order, of the values of the
@@ -440,13 +449,14 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
         acc = mfma(as_half8(word_a), as_half8(word_b), acc);
         accm = mfma(as_half8(word_a), as_half8(word_c), accm);
         word_a.x = *(const uint32_t*)(sum0 + off + 4 * B);
+        word_c.x = sc.mins_low;
         accm = mfma(as_half8(word_a), as_half8(word_c), accm);
         float v[kRegs];
 #pragma unroll
         for (int r = 0; r < kRegs; r++) {
-            float full = add_other_half(acc[r]), m = accm[r];
+            float full = add_low_rows(acc[r]), m = accm[r];
             if constexpr (BP < 4) {
-                const float full2 = add_other_half(acc[r + 2]);
+                const float full2 = add_low_rows(acc[r + 2]);
                 full = upper ? full2 : full;
                 m = upper ? accm[r + 2] : m;
             }
@@ -636,11 +646,13 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
                     lo[i][j] = mfma(as_half8(word_l), as_half8(word_w), lo[i][j]);
                     word_w.x = sc[i].mins;
                     floatx4 m = mfma(as_half8(word_h), as_half8(word_w), floatx4{0.f, 0.f, 0.f, 0.f});
+                    word_w.x = sc[i].mins_low;
                     m = mfma(as_half8(word_l), as_half8(word_w), m);
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        total[i][j][r] =
-                            __builtin_fmaf(Q4k::value(sc[i], hi[i][j][r] + lo[i][j][r], m[r]), inv[r], total[i][j][r]);
+                        total[i][j][r] = __builtin_fmaf(
+                            Q4k::value(sc[i], __builtin_fmaf(lo[i][j][r], kLowTerm, hi[i][j][r]), m[r]), inv[r],
+                            total[i][j][r]);
                 }
             }
         }

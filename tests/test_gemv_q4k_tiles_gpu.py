@@ -1,11 +1,11 @@
 """Q4_K products at the edges of the kernels' tiles (gpu).
 
-Row counts around the 8- and 16-row units and the 32- to 384-row tiles, row
-lengths of 1 to 56 blocks (fewer blocks than a step takes, blocks that do not
-divide among the wavefronts or the four sums, rows whose converted inputs do
-not fit the LDS) and input counts around 8, 16 and 32.  Every input's output is
-checked against the float64 dequantise-then-dot and must equal the single
-call's bit for bit.
+Row counts around the 8- and 16-row units and the smallest tiles, row lengths
+of 1 to 208 blocks (fewer blocks than a step takes, blocks that do not divide
+among the wavefronts or the four sums, rows whose converted inputs do not fit
+the LDS) and input counts around 8, 16 and 32; then each of the tiles.  Outputs
+are checked against the float64 dequantise-then-dot and must equal those of
+single or eight-input calls bit for bit.
 
 Tolerance: inputs are carried to within 2^-23 and products summed in f32, so
 per output |error| <= c 2^-23 sum|w x| with a small c (the sums' roundings add
@@ -33,6 +33,16 @@ def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
+def terms(w, n_rows, n_cols):
+    """|d scale q| + |dmin min| of every weight, float64."""
+    total = 0.0
+    for field in (0, 2):  # without d, without dmin
+        part = w.reshape(-1, 144).copy()
+        part[:, field:field + 2] = 0
+        total = total + np.abs(W.q4k_dequant_np(part, n_rows, n_cols).astype(np.float64))
+    return total.reshape(n_rows, n_cols)
+
+
 @pytest.mark.parametrize("n_rows,n_cols,batch", CASES)
 def test_q4k_tile_edges(gpu, n_rows, n_cols, batch):
     w = W.q4k_random_weights(n_rows, n_cols, seed=n_rows + n_cols)
@@ -52,11 +62,7 @@ def test_q4k_tile_edges(gpu, n_rows, n_cols, batch):
     assert torch.isnan(out[:, n_rows:]).all()  # stride padding untouched
     deq = W.q4k_dequant_np(w, n_rows, n_cols).astype(np.float64).reshape(n_rows, n_cols)
     ref = x.astype(np.float64) @ deq.T
-    blocks = w.reshape(n_rows, -1, 144)
-    d = blocks[:, :, 0:4].copy().view(np.float16).astype(np.float64)  # d, dmin
-    # at most 15 * 63 d + 63 dmin per weight of the block
-    most = np.repeat(945 * np.abs(d[..., 0]) + 63 * np.abs(d[..., 1]), 256, axis=1)
-    bound = 4 * 2.0**-23 * (np.abs(x).astype(np.float64) @ most.T)
+    bound = 4 * 2.0**-23 * (np.abs(x).astype(np.float64) @ terms(w, n_rows, n_cols).T)
     got = out[:, :n_rows].cpu().numpy().astype(np.float64)
     assert np.all(np.abs(got - ref) <= bound), np.max(np.abs(got - ref) / bound)
 
@@ -65,8 +71,7 @@ def test_q4k_tile_edges(gpu, n_rows, n_cols, batch):
 def test_q4k_input_extremes(gpu, n_cols, batch):
     """Zeros, values at either end of f32 and a power-of-two ladder are scaled
     within their block, blocks and inputs apart from each other; an infinity or
-    a NaN makes its own input's outputs NaN (as inf - inf and 0 * inf do in the
-    formula) and no other's."""
+    a NaN makes every output of its own input NaN and none of another's."""
     n_rows = 37
     w = W.q4k_random_weights(n_rows, n_cols, seed=5)
     rng = np.random.default_rng(6)
@@ -125,3 +130,37 @@ def test_q4k_every_tile(gpu, n_rows, batch, blocks):
     bound = 8 * 2.0**-23 * (np.abs(x).astype(np.float64) @ np.abs(deq).T)
     got = out[:, torch.from_numpy(rows).cuda()].cpu().numpy()
     assert np.all(np.abs(got - ref) <= bound), np.max(np.abs(got - ref) / bound)
+
+
+@pytest.mark.parametrize("index", [3, 40, 131, 255])
+@pytest.mark.parametrize("batch", [1, 3, 20])
+def test_q4k_large_values_under_zero_weights(gpu, batch, index):
+    """One value of each block 2^6 to 2^24 times the others, where every weight
+    is zero, through zero scale and min: the others keep their precision.
+
+    The roundings of f32 sums are independent of each other and 2^-24 of terms
+    or of sums of their size, so the errors' norm is c 2^-24 of the norm of the
+    terms, for which |w x| stands; c = 6 (three roundings a term, twice)."""
+    n_rows, n_cols = 300, 2048
+    w = W.q4k_random_weights(n_rows, n_cols, seed=index)
+    b = w.reshape(-1, 144)
+    sub = index // 32
+    for field in (0, 4):  # the sub-block's scale, min
+        if sub < 4:
+            b[:, 4 + field + sub] &= 0xc0
+        else:
+            b[:, 8 + sub] &= 0xf0 if field == 0 else 0x0f
+            b[:, field + sub] &= 0x3f
+    deq = W.q4k_dequant_np(w, n_rows, n_cols).astype(np.float64).reshape(n_rows, n_cols)
+    assert not np.any(deq[:, index::256])
+    rng = np.random.default_rng(batch)
+    for bits in (6, 10, 16, 20, 24):
+        x = rng.standard_normal((batch, n_cols)).astype(np.float32)
+        ref = x.astype(np.float64) @ deq.T
+        norm = np.sqrt(np.sum(x.astype(np.float64)**2 @ (deq**2).T))
+        x[:, index::256] = np.float32(1.37 * 2.0**bits)
+        out = torch.full((batch, n_rows), float("nan"), device="cuda")
+        gpu.gemv_q4k_batched(dev(w), dev(x), out, n_rows, n_cols)
+        torch.cuda.synchronize()
+        err = np.linalg.norm(out.cpu().numpy() - ref)
+        assert err <= 6 * 2.0**-24 * norm, (bits, err / norm)
