@@ -11,10 +11,13 @@
 // Arithmetic.  Every product runs on v_mfma_f32_16x16x32_f16, inputs as the
 // 16 rows of A and weight rows as the 16 columns of B, with operands that
 // hold the f32 product exactly but for the last bit of x:
-//  * scale * (q - 8), at most 504 in magnitude, is exact in binary16, so the
-//    block's d multiplies one f32 sum per block; 8 * scale and dmin * min
-//    multiply the sums of x per sub-block (the offset of 8 keeps the first sum
-//    as small as the result: without it the error was 1.5 times larger);
+//  * scale * (q - z), at most 945 in magnitude, is exact in binary16, so the
+//    block's d multiplies one f32 sum per block; scale * z and dmin * min
+//    multiply the sums of x per sub-block.  z = round(dmin * min / (d * scale))
+//    makes these operands about as small as the weights (z = 0 throughout: 1.5
+//    times the error), and zero where a weight is zero: a value of x that no
+//    weight takes up, however large, costs the others nothing (a fixed z = 8
+//    under min = 0 put 2e-5 of the output's norm in it for a value of 2^10);
 //  * each input's 256 values of a block are scaled by the power of two that
 //    brings their largest magnitude into [2^14, 2^15) and split into two
 //    binary16 terms, x = hi + lo 2^-11, which hold it to within 2^-23 of x or
@@ -24,10 +27,10 @@
 // A block's value for one (row, input) is a chain of eight K steps, and an
 // output is the sum of kSumWays sums of its blocks' values, whichever kernel,
 // tile or wavefront computed them: single, multi-matrix and batched calls
-// give the same bits.  Against float64 the outputs are off by 1.6e-7 to 1.7e-7
+// give the same bits.  Against float64 the outputs are off by 1.6e-7 to 1.8e-7
 // of their norm for N(0, 1) inputs (256 to 14336 columns; f32 FMAs in runs of
-// 16 were 1.8e-7 to 2.1e-7), and as much beside a value 2^24 times the others
-// under zero scales.
+// 16 were 1.8e-7 to 2.1e-7), and as much beside a value 2^28 times the others
+// that meets zero weights.
 //
 // Two kernels.  gemv_split_kernel (up to eight inputs): the wavefronts of a
 // workgroup take the blocks of 16 rows among them, each converting the inputs
@@ -61,16 +64,8 @@ __device__ __forceinline__ uint32_t as_word(halfx2 h) { return __builtin_bit_cas
 __device__ __forceinline__ halfx8 as_half8(u32x4 w) { return __builtin_bit_cast(halfx8, w); }
 __device__ __forceinline__ halfx2 splat2(_Float16 h) { return halfx2{h, h}; }
 
-// 1024 + n in each half of a word holding two integers n < 1024
+// The high bytes of two halves 1024 + n, n < 256
 constexpr uint32_t kHalf1024 = 0x64006400u;
-
-// The same constant kept in a vector register: v_and_or_b32 takes one scalar
-// operand, which its mask is.
-__device__ __forceinline__ uint32_t half1024_reg() {
-    uint32_t k = kHalf1024;
-    asm("" : "+v"(k));
-    return k;
-}
 
 // What the low terms of x count: they are kept 2^11 times larger, so that
 // they are normal binary16 numbers wherever the high terms are.
@@ -91,12 +86,12 @@ struct Q4k {
     struct Raw {
         u32x4 hdr, qa, qb;
     };
-    // Scales of the two sub-blocks for the low nibbles' and the high nibbles'
-    // weights, scales and mins as operands of the sums of x (the mins also for
-    // their low terms), d and dmin.
+    // Factors and offsets of the two sub-blocks for the low nibbles' and the
+    // high nibbles' weights; scale * offset and the mins as operands of the
+    // sums of x (the mins also for their low terms); d and dmin.
     struct Scales {
-        halfx2 s_lo, s_hi, c_hi;
-        uint32_t scales, mins, mins_low;
+        halfx2 s_lo, o_lo, s_hi, o_hi;
+        uint32_t offsets, mins, mins_low;
         float d, dmin;
     };
     __device__ static int x_offset(int s, int g) { return 64 * g + 4 * s; }
@@ -108,35 +103,43 @@ struct Q4k {
     // unpack_scales_q4k for sub-blocks 2g and 2g+1, two bytes at a time: the
     // 6-bit fields of sub-blocks 0-3 are whole bytes, those of 4-7 a nibble
     // and two bits (masks, so that the lanes do not part)
-    __device__ __forceinline__ static void scales(const Raw& r, int g, uint32_t k1024, Scales& c) {
+    __device__ __forceinline__ static void scales(const Raw& r, int g, Scales& c) {
         const int k = 16 * (g & 1);
         const uint32_t whole = g < 2 ? 0x3f3fu : 0u, nib = g < 2 ? 0u : 0x0f0fu, two = g < 2 ? 0u : 0x3030u;
         const uint32_t a = r.hdr.y >> k, b = r.hdr.z >> k, e = r.hdr.w >> k;
         const uint32_t sc = (a & whole) | (e & nib) | ((a >> 2) & two);
         const uint32_t mn = (b & whole) | ((e >> 4) & nib) | ((b >> 2) & two);
         // bytes 0 and 1 as the low bytes of two halves 1024 + n
-        const halfx2 s = as_half2(__builtin_amdgcn_perm(k1024, sc, 0x07010700u)) - splat2(1024);
-        const halfx2 m = as_half2(__builtin_amdgcn_perm(k1024, mn, 0x07010700u)) - splat2(1024);
-        // low nibbles, masked in place, are the binary16 denormals q 2^-24;
-        // high nibbles under the exponent of 1024 are 1024 + 16 q = 16 (64 + q)
+        const halfx2 s = as_half2(__builtin_amdgcn_perm(kHalf1024, sc, 0x07010700u)) - splat2(1024);
+        const halfx2 m = as_half2(__builtin_amdgcn_perm(kHalf1024, mn, 0x07010700u)) - splat2(1024);
+        const float d = f16_bits_to_f32(r.hdr.x), dmin = f16_bits_to_f32(r.hdr.x >> 16);
+        // z = dmin * min / (d * scale) to the nearest integer within 0 .. 15
+        // (any would do: quotients of zeros, infinities and NaNs end in there too)
+        halfx2 z = m * halfx2{(_Float16)__builtin_amdgcn_rcph(s.x), (_Float16)__builtin_amdgcn_rcph(s.y)} *
+                   splat2((_Float16)(dmin * __builtin_amdgcn_rcpf(d)));
+        z = __builtin_elementwise_min(__builtin_elementwise_max(z, splat2(0)), splat2(15));
+        z = (z + splat2(1024)) - splat2(1024);
+        const halfx2 sz = s * z;
+        // nibbles masked in place are the binary16 denormals q 2^-24 (low) and
+        // q 2^-20 (high)
         c.s_lo = splat2(s.x) * splat2(1024);
-        c.s_hi = splat2(s.y) * splat2((_Float16)(1.0 / 262144));
-        c.c_hi = splat2(s.y) * splat2((_Float16)(-72.0 / 16384));
-        c.scales = as_word(s * splat2((_Float16)(1.0 / 64)));
+        c.s_hi = splat2(s.y) * splat2(64);
+        c.o_lo = splat2(sz.x) * splat2((_Float16)(-1.0 / 16384));
+        c.o_hi = splat2(sz.y) * splat2((_Float16)(-1.0 / 16384));
+        c.offsets = as_word(sz * splat2((_Float16)(1.0 / 512)));
         c.mins = as_word(m);
         c.mins_low = as_word(m * splat2((_Float16)kLowTerm));
-        c.d = f16_bits_to_f32(r.hdr.x) * 16384.f;
-        c.dmin = f16_bits_to_f32(r.hdr.x >> 16) * 32.f;
+        c.d = d * 16384.f;
+        c.dmin = dmin * 32.f;
     }
-    // scale * (q - 8) * 2^-14, exact
-    __device__ __forceinline__ static halfx8 weights(const Raw& r, const Scales& c, uint32_t k1024, int s) {
+    // scale * (q - z) * 2^-14, exact
+    __device__ __forceinline__ static halfx8 weights(const Raw& r, const Scales& c, int s) {
         const uint32_t q = s < 4 ? r.qa[s] : r.qb[s - 4];
         const uint32_t o = q >> 8;
-        const halfx2 eight = as_half2(0x00080008u);  // 8 * 2^-24
-        const u32x4 v = {as_word((as_half2(q & 0x000f000fu) - eight) * c.s_lo),
-                         as_word((as_half2(o & 0x000f000fu) - eight) * c.s_lo),
-                         as_word(__builtin_elementwise_fma(as_half2((q & 0x00f000f0u) | k1024), c.s_hi, c.c_hi)),
-                         as_word(__builtin_elementwise_fma(as_half2((o & 0x00f000f0u) | k1024), c.s_hi, c.c_hi))};
+        const u32x4 v = {as_word(__builtin_elementwise_fma(as_half2(q & 0x000f000fu), c.s_lo, c.o_lo)),
+                         as_word(__builtin_elementwise_fma(as_half2(o & 0x000f000fu), c.s_lo, c.o_lo)),
+                         as_word(__builtin_elementwise_fma(as_half2(q & 0x00f000f0u), c.s_hi, c.o_hi)),
+                         as_word(__builtin_elementwise_fma(as_half2(o & 0x00f000f0u), c.s_hi, c.o_hi))};
         return as_half8(v);
     }
     // The block's value of one (row, input), of the scaled input, from its
@@ -320,7 +323,6 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
     const long long row_bytes = (long long)nb * Q4k::kBlockBytes;
     constexpr int kBlk = split_block_bytes(B);
     float* vals = (float*)(lds + (EACH_STEP ? P * KB : nb) * kBlk);
-    const uint32_t k1024 = half1024_reg();
     const int row_n = n % R, blk_n = n / R;  // this lane's row of the unit and block of the group
 
     // the matrix of unit u and its first unit
@@ -434,17 +436,17 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
         const int b0 = (kp + P * pass) * KB;
         const int off = (EACH_STEP ? blk_a : min(b0 + blk_a, nb - 1)) * kBlk;
         Q4k::Scales sc;
-        Q4k::scales(cur, g, k1024, sc);
+        Q4k::scales(cur, g, sc);
         floatx4 acc = {0.f, 0.f, 0.f, 0.f}, accm = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int st = 0; st < 8; st++) {
             const halfx8 xv = as_half8(*(const u32x4*)(op0 + off + st * 128 * B));
-            acc = mfma(xv, Q4k::weights(cur, sc, k1024, st), acc);
+            acc = mfma(xv, Q4k::weights(cur, sc, st), acc);
         }
-        // the scales' term as the weights' (hi and lo rows), the mins' in turn
+        // the offsets' term as the weights' (hi and lo rows), the mins' in turn
         // into the rows of hi
         word_a.x = *(const uint32_t*)(sum0 + off);
-        word_b.x = sc.scales;
+        word_b.x = sc.offsets;
         word_c.x = sc.mins;
         acc = mfma(as_half8(word_a), as_half8(word_b), acc);
         accm = mfma(as_half8(word_a), as_half8(word_c), accm);
@@ -545,7 +547,6 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
     const int in0 = ((int)blockIdx.x % a.in_tiles) * TM;
     const int row0 = ((int)blockIdx.x / a.in_tiles) * (RW * RT * 16) + (wave % RW) * RT * 16;
     const long long row_bytes = (long long)nb * Q4k::kBlockBytes;
-    const uint32_t k1024 = half1024_reg();
     const uint8_t* wp[RT];
 #pragma unroll
     for (int i = 0; i < RT; i++) wp[i] = a.w + min(row0 + 16 * i + n, a.rows - 1) * row_bytes;
@@ -611,7 +612,7 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
         if (KS == 1 || b < nb) {
             Q4k::Scales sc[RT];
 #pragma unroll
-            for (int i = 0; i < RT; i++) Q4k::scales(cur[i], g, k1024, sc[i]);
+            for (int i = 0; i < RT; i++) Q4k::scales(cur[i], g, sc[i]);
             floatx4 hi[RT][MT], lo[RT][MT];
 #pragma unroll
             for (int i = 0; i < RT; i++)
@@ -621,7 +622,7 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
             for (int st = 0; st < 8; st++) {
                 halfx8 w[RT];
 #pragma unroll
-                for (int i = 0; i < RT; i++) w[i] = Q4k::weights(cur[i], sc[i], k1024, st);
+                for (int i = 0; i < RT; i++) w[i] = Q4k::weights(cur[i], sc[i], st);
 #pragma unroll
                 for (int j = 0; j < MT; j++) {
                     const halfx8 xh = as_half8(X.x[j][0][st][lane]), xl = as_half8(X.x[j][1][st][lane]);
@@ -641,7 +642,7 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
                 word_l.x = X.sums[j][1][g][n];
 #pragma unroll
                 for (int i = 0; i < RT; i++) {
-                    word_w.x = sc[i].scales;
+                    word_w.x = sc[i].offsets;
                     hi[i][j] = mfma(as_half8(word_h), as_half8(word_w), hi[i][j]);
                     lo[i][j] = mfma(as_half8(word_l), as_half8(word_w), lo[i][j]);
                     word_w.x = sc[i].mins;

@@ -133,10 +133,12 @@ def test_q4k_every_tile(gpu, n_rows, batch, blocks):
 
 
 @pytest.mark.parametrize("index", [3, 40, 131, 255])
+@pytest.mark.parametrize("zero", ["scale and min", "min and nibble"])
 @pytest.mark.parametrize("batch", [1, 3, 20])
-def test_q4k_large_values_under_zero_weights(gpu, batch, index):
-    """One value of each block 2^6 to 2^24 times the others, where every weight
-    is zero, through zero scale and min: the others keep their precision.
+def test_q4k_large_values_under_zero_weights(gpu, batch, zero, index):
+    """One value of each block 2^6 to 2^28 times the others, where every weight
+    is zero, through zero scale and min or zero min and nibble: the others keep
+    their precision.
 
     The roundings of f32 sums are independent of each other and 2^-24 of terms
     or of sums of their size, so the errors' norm is c 2^-24 of the norm of the
@@ -144,17 +146,19 @@ def test_q4k_large_values_under_zero_weights(gpu, batch, index):
     n_rows, n_cols = 300, 2048
     w = W.q4k_random_weights(n_rows, n_cols, seed=index)
     b = w.reshape(-1, 144)
-    sub = index // 32
-    for field in (0, 4):  # the sub-block's scale, min
+    sub, i = index // 32, index % 32
+    for field in (4,) if zero == "min and nibble" else (0, 4):  # the sub-block's scale, min
         if sub < 4:
             b[:, 4 + field + sub] &= 0xc0
         else:
             b[:, 8 + sub] &= 0xf0 if field == 0 else 0x0f
             b[:, field + sub] &= 0x3f
+    if zero == "min and nibble":
+        b[:, 16 + 32 * (sub // 2) + i] &= 0x0f if sub % 2 else 0xf0
     deq = W.q4k_dequant_np(w, n_rows, n_cols).astype(np.float64).reshape(n_rows, n_cols)
     assert not np.any(deq[:, index::256])
     rng = np.random.default_rng(batch)
-    for bits in (6, 10, 16, 20, 24):
+    for bits in (6, 10, 16, 20, 24, 28):
         x = rng.standard_normal((batch, n_cols)).astype(np.float32)
         ref = x.astype(np.float64) @ deq.T
         norm = np.sqrt(np.sum(x.astype(np.float64)**2 @ (deq**2).T))
