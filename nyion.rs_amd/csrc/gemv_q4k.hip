@@ -47,6 +47,8 @@
 // 1320 and 39.
 #include "gemv.hpp"
 
+#include <limits.h>
+
 #include <algorithm>
 
 namespace nyion {
@@ -201,11 +203,11 @@ struct XTerms {
 // denormal high term leaves (kept out of v_fma_mix, which issues at a quarter
 // of the rate of a subtraction).
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
-    const halfx2 h = {(_Float16)a, (_Float16)b};
-    float ha = (float)h.x, hb = (float)h.y;
+    hi = as_word(halfx2{(_Float16)a, (_Float16)b});
+    asm("" : "+v"(hi));
+    float ha = (float)as_half2(hi).x, hb = (float)as_half2(hi).y;
     asm("" : "+v"(ha));
     asm("" : "+v"(hb));
-    hi = as_word(h);
     lo = as_word(halfx2{(_Float16)((a - ha) * (1.f / kLowTerm)), (_Float16)((b - hb) * (1.f / kLowTerm))});
 }
 
@@ -251,7 +253,15 @@ __device__ __forceinline__ float add_low_rows(float x) {
 // An output is the sum of kSumWays sums, in order, of the values of the
 // blocks k, k + kSumWays, ...
 constexpr int kSumWays = 4;
-__device__ __forceinline__ float sum_ways(const float (&s)[kSumWays]) { return ((s[0] + s[1]) + s[2]) + s[3]; }
+
+// The sum of a quad's values in order, in its first lane (the quad's lanes
+// all active).
+__device__ __forceinline__ float sum_quad(float x) {
+    const uint32_t v = __float_as_uint(x);
+    x += __uint_as_float(dpp<0x55>(v));  // quad_perm [1,1,1,1]
+    x += __uint_as_float(dpp<0xaa>(v));  // quad_perm [2,2,2,2]
+    return x + __uint_as_float(dpp<0xff>(v));
+}
 
 __device__ __forceinline__ floatx4 mfma(const halfx8& a, const halfx8& b, const floatx4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -275,12 +285,14 @@ struct GemvMat {
     const uint8_t* w;  // [rows][nb * block bytes]
     float* out;        // [n_inputs][out_stride]
     int rows;
-    int unit_end;  // units of the matrices up to this one
+    int unit0;  // its first unit (INT_MAX: no such matrix)
 };
 
 struct GemvSplitArgs {
     GemvMat mat[kGemvMaxMats];
-    int n_mats;
+    int units;       // of all matrices
+    int full, rest;  // groups of blocks per wavefront, one more for the first `rest`
+    int waves;       // of a workgroup
     const float* x;  // [n_inputs][x_stride]
     long long x_stride;
     long long out_stride;
@@ -313,44 +325,49 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
     static_assert(B <= BP, "inputs of a step");
     const int lane = threadIdx.x & 63;
     const int kp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int P = (int)blockDim.x >> 6;
+    const int P = a.waves;
     const int n = lane & 15, g = lane >> 4;
     const int nb = a.nb, last_in = a.n_inputs - 1;
-    const int ng = (nb + KB - 1) / KB;        // groups of KB blocks
-    const int npass = (ng - kp + P - 1) / P;  // this wavefront's groups kp, kp + P, ... (>= 1: P <= ng)
+    const int npass = a.full + (kp < a.rest);  // this wavefront's groups kp, kp + P, ... of KB blocks
     const int first = (int)blockIdx.x, stride = (int)gridDim.x;  // units first, first + stride, ...
-    const int U = a.mat[a.n_mats - 1].unit_end;
+    const int U = a.units;
     const long long row_bytes = (long long)nb * Q4k::kBlockBytes;
     constexpr int kBlk = split_block_bytes(B);
     float* vals = (float*)(lds + (EACH_STEP ? P * KB : nb) * kBlk);
     const int row_n = n % R, blk_n = n / R;  // this lane's row of the unit and block of the group
 
-    // the matrix of unit u and its first unit
-    auto mat_of = [&](int u, int& u0) __attribute__((always_inline)) {
-        int m = 0;
-        u0 = 0;
+    // the matrix of unit u, selected in scalar registers: an indexed load of
+    // the arguments is one more round trip ahead of the weights, and of the
+    // outputs behind the sums
+    auto mat_of = [&](int u) __attribute__((always_inline)) {
+        GemvMat m = a.mat[0];
 #pragma unroll
-        for (int i = 0; i < kGemvMaxMats - 1; i++)
-            if (i + 1 < a.n_mats && u >= a.mat[i].unit_end) {
-                m = i + 1;
-                u0 = a.mat[i].unit_end;
-            }
+        for (int i = 1; i < kGemvMaxMats; i++) {
+            const uint8_t* const w = a.mat[i].w;
+            float* const out = a.mat[i].out;
+            const int rows = a.mat[i].rows, unit0 = a.mat[i].unit0;
+            const bool in = u >= unit0;
+            m.w = in ? w : m.w;
+            m.out = in ? out : m.out;
+            m.rows = in ? rows : m.rows;
+            m.unit0 = in ? unit0 : m.unit0;
+        }
         return m;
     };
     // rows past the matrix repeat its last, blocks past the row its last
     auto load_w = [&](int u, int pass, Q4k::Raw& r) __attribute__((always_inline)) {
-        int u0;
-        const int m = mat_of(u, u0);
-        const int row = min((u - u0) * R + row_n, a.mat[m].rows - 1);
+        const GemvMat m = mat_of(u);
+        const int row = min((u - m.unit0) * R + row_n, m.rows - 1);
         const int b = min((kp + P * pass) * KB + blk_n, nb - 1);
-        Q4k::load(a.mat[m].w + row * row_bytes + (long long)b * Q4k::kBlockBytes, g, r);
+        Q4k::load(m.w + row * row_bytes + (long long)b * Q4k::kBlockBytes, g, r);
     };
 
     // inputs, two (block, input) pairs at a time, one per half wavefront
     // (inputs past the last repeat it, and an odd last pair is done twice)
     const int s = lane & 7, gx = (lane >> 3) & 3, half = lane >> 5;
     auto load_pair = [&](int b, int in) __attribute__((always_inline)) {
-        return load_x(a.x + min(in, last_in) * a.x_stride + (long long)b * kKqBlockElems, s, gx);
+        const float* x = B == 1 ? a.x : a.x + min(in, last_in) * a.x_stride;
+        return load_x(x + (long long)b * kKqBlockElems, s, gx);
     };
     auto store_pair = [&](const XShare& xs, uint8_t* base, int in) __attribute__((always_inline)) {
         const XTerms t = split_x(xs);
@@ -380,23 +397,33 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
         load_w(first, 0, raw[0]);
     } else {
         // all of this wavefront's blocks; the first weights are requested
-        // between the loads and the conversion of the first pairs
+        // behind the loads of the first pairs and ahead of their conversion.
+        // The fence holds them there: loads return in order, and with the
+        // weights first the conversion began only when they had come from HBM
+        // (88 launches of 256 to 11264 rows, replayed: 493 -> 414 us with the
+        // matrices and passes below out of the way too)
         const int pairs = npass * kPairs;
-        auto block_of = [&](int c) __attribute__((always_inline)) {
-            const int k = c / B;
-            return min((kp + P * (k / KB)) * KB + k % KB, nb - 1);
+        auto block_of = [&](unsigned c) __attribute__((always_inline)) {
+            const unsigned k = c / B;
+            return min((kp + P * (int)(k / KB)) * KB + (int)(k % KB), nb - 1);
         };
         auto load_at = [&](int i) __attribute__((always_inline)) {
             const int c = min(i, pairs - 1);
             return load_pair(block_of(c), c % B);
         };
-        XShare cx[2] = {load_at(half), load_at(2 + half)};
-        load_w(first, 0, raw[0]);
-        for (int i = 0; i < pairs; i += 2) {
+        auto store_at = [&](const XShare& x, int i) __attribute__((always_inline)) {
             const int c = min(i + half, pairs - 1);
-            store_pair(cx[0], lds + block_of(c) * kBlk, c % B);
-            cx[0] = cx[1];
-            if (i + 4 < pairs) cx[1] = load_at(i + 4 + half);
+            store_pair(x, lds + block_of(c) * kBlk, c % B);
+        };
+        XShare cur = load_at(half), next;
+        if (pairs > 2) next = load_at(2 + half);
+        asm volatile("" ::: "memory");
+        load_w(first, 0, raw[0]);
+        store_at(cur, 0);
+        for (int i = 2; i < pairs; i += 2) {
+            cur = next;
+            if (i + 2 < pairs) next = load_at(i + 2 + half);
+            store_at(cur, i);
         }
     }
 
@@ -473,21 +500,18 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
         if (++pass < npass) return;
         pass = 0;
         __syncthreads();  // the buffers alternate, so one barrier per unit suffices
-        for (int o = threadIdx.x; o < R * B; o += (int)blockDim.x) {
+        // one thread per output and sum, the four of an output in a quad (4096
+        // x 14336 11.9 -> 11.7 us against one thread per output)
+        for (int t = threadIdx.x; t < R * B * kSumWays; t += 64 * P) {
+            const int o = t / kSumWays;
             const float* w = vals + par * nb * B * R + o;
-            float sum[kSumWays] = {};
-            int i = 0;
-#pragma unroll 2
-            for (; i + kSumWays <= nb; i += kSumWays)
-#pragma unroll
-                for (int k = 0; k < kSumWays; k++) sum[k] += w[(i + k) * B * R];
-#pragma unroll
-            for (int k = 0; k < kSumWays - 1; k++)
-                if (i + k < nb) sum[k] += w[(i + k) * B * R];
-            int u0;
-            const int m = mat_of(u, u0);
-            const int row = (u - u0) * R + o % R;
-            if (row < a.mat[m].rows && o / R <= last_in) a.mat[m].out[o / R * a.out_stride + row] = sum_ways(sum);
+            float sum = 0.f;
+#pragma unroll 4
+            for (int i = t % kSumWays; i < nb; i += kSumWays) sum += w[i * B * R];
+            sum = sum_quad(sum);
+            const GemvMat m = mat_of(u);
+            const int row = (u - m.unit0) * R + o % R;
+            if (t % kSumWays == 0 && row < m.rows && o / R <= last_in) m.out[o / R * a.out_stride + row] = sum;
         }
         par ^= 1;
         u += stride;
@@ -753,8 +777,16 @@ static SplitShape split_shape(int nb, int units, int B, int R) {
 template <int B, int R>
 static int launch_split_br(GemvSplitArgs& a, int cus, hipStream_t st) {
     int units = 0;
-    for (int m = 0; m < a.n_mats; m++) a.mat[m].unit_end = units += ceil_div(a.mat[m].rows, R);
+    for (int m = 0; m < kGemvMaxMats; m++) {
+        a.mat[m].unit0 = a.mat[m].rows > 0 ? units : INT_MAX;
+        units += ceil_div(a.mat[m].rows, R);
+    }
+    a.units = units;
     const SplitShape sh = split_shape(a.nb, units, B, R);
+    const int groups = ceil_div(a.nb, 16 / R);
+    a.waves = sh.waves;
+    a.full = groups / sh.waves;
+    a.rest = groups % sh.waves;
     // resident workgroups: four or (one input) five wavefronts per SIMD
     const int cap = std::max(1, std::min((B > 1 ? 16 : 20) / sh.waves, kLdsPerCu / sh.lds)) * cus;
     static std::atomic<int> allowed[2][kMaxDevices];
@@ -852,7 +884,6 @@ int gemv_q4k_launch(const uint8_t* const* ws, const float* x, long long x_stride
             a.mat[m] = GemvMat{ws[m], outs[m], row_counts[m], 0};
             rows += row_counts[m];
         }
-        a.n_mats = n_mats;
         a.nb = nb;
         a.x = x;
         a.x_stride = x_stride;
