@@ -274,16 +274,17 @@ __device__ __forceinline__ void write_chunk_rows(const PrefillArgs& a, int g, in
     const int r0 = rbg * a.rb_per_wg * 32;
     const int r1 = min(a.n, r0 + a.rb_per_wg * 32);
     float vmax = 0.f;
-    for (int i = tid; i < (r1 - r0) * VEC; i += threads) {
-        const int r = r0 + i / VEC, x = i % VEC;
-        if (!a.kv_write)
-            vmax = fmaxf(vmax, v_absmax(*(const uint2*)(a.v + ((long long)r * a.n_kv_heads + g) * D + 4 * x)));
-        else if (a.kv_dtype == NYION_KV_Q4_20B)
-            vmax = fmaxf(vmax, write_kv_q4_vec(a.kvw, r, g, x));  // 8 lanes per group: VEC is a multiple
-        else
-            vmax = fmaxf(vmax, a.kv_dtype == NYION_KV_F16 ? write_kv_vec<true>(a.kvw, r, g, x)
-                                                          : write_kv_vec<false>(a.kvw, r, g, x));
-    }
+    auto each = [&](auto write) __attribute__((always_inline)) {
+        for (int i = tid; i < (r1 - r0) * VEC; i += threads) vmax = fmaxf(vmax, write(r0 + i / VEC, i % VEC));
+    };
+    if (!a.kv_write)
+        each([&](int r, int x) { return v_absmax(*(const uint2*)(a.v + ((long long)r * a.n_kv_heads + g) * D + 4 * x)); });
+    else if (a.kv_dtype == NYION_KV_Q4_20B)
+        each([&](int r, int x) { return write_kv_q4_vec(a.kvw, r, g, x); });  // 8 lanes per group: VEC is a multiple
+    else if (a.kv_dtype == NYION_KV_F16)
+        each([&](int r, int x) { return write_kv_vec<true>(a.kvw, r, g, x); });
+    else
+        each([&](int r, int x) { return write_kv_vec<false>(a.kvw, r, g, x); });
     report_range(a.kvw.status, vmax >= 65520.f, kRangePrefillV);
 }
 
@@ -872,9 +873,8 @@ static int launch_prefill(PrefillArgs& a, hipStream_t st, bool& split) {
     // 128).  With a history the split kernel also saves the launch that
     // checks its V, which outweighs the merge at any length: one row after
     // 128 12.5 / 9.7 (d 64) and 13.4 / 10.2 (d 128).
-    constexpr int kCus = 256;
     const int tiles = (a.n_hist + BN - 1) / BN + (a.n + BN - 1) / BN;
-    split = prefill_items(a, GW) <= kCus && (tiles >= 2 * NG || a.n_hist > 0);
+    split = prefill_items(a, GW) <= device_cu_count() && (tiles >= 2 * NG || a.n_hist > 0);
     if (split) return launch_prefill_split<D, GW, NG>(a, st);
     const long long items = prefill_items(a, prefill_threads<D>() / 64);
     if (items > (1LL << 30)) return set_error(NYION_ERR_UNSUPPORTED, "prefill: %lld work items", items);
