@@ -123,7 +123,7 @@ struct DecodeArgs {
     int direct;        // > 0: direct partition, pieces per segment (else stream-K)
     int seg_tiles;     // direct: host bound on the tiles of one segment
     int ragged_min;    // > 0: direct, pieces in proportion to the lengths
-                       // (ragged_pieces), this many tiles or more each
+                       // (ragged_piece), this many tiles or more each
     int spec_len;      // window mode: the host's max_ctx, whose window start a
                        // walk's block-table loads may assume before the
                        // length arrives (0: none)
@@ -196,7 +196,6 @@ __device__ __forceinline__ Extent extent_of(const DecodeArgs& a, int2 v) {
     return a.mode == MODE_LIST ? seq_extent<ALIGNED>(a, 0, 0, v.x) : seq_extent<ALIGNED>(a, v.x, v.y, 0);
 }
 
-// Extent of sequence b as seen by one thread (no uniformity assumed).
 // Inclusive prefix sum over the wavefront (every lane active), on DPP row
 // shifts and row broadcasts.
 __device__ __forceinline__ int wave_scan(int x) {
@@ -214,12 +213,12 @@ __device__ __forceinline__ int wave_scan(int x) {
 // equal cut a launch lasts as long as the longest sequence's pieces while the
 // workgroups of the others idle (8 binary16 sequences of 300-3000 tokens, 32/8
 // heads of 128: 23.7 -> 19.7 us; of 4000-16000 77.5 -> 62.5; f32 39.0 -> 30.9;
-// equal lengths of 3000: 25.7 -> 25.4).  Every segment is cut into ceil(tiles / c) pieces (at
-// least one), with one c for all, the smallest of a few candidates at which
-// the batch's pieces number at most the grid: from the even share of all
-// tiles (exact when the lengths are equal: the host's own cut) towards the
-// bound that always fits.  Each wavefront computes it for itself, lane l
-// holding sequence l (at most 64), without barriers.
+// equal lengths of 3000: 25.7 -> 25.4).  Every segment is cut into
+// ceil(tiles / c) pieces (at least one), with one c for all, the smallest of a
+// few candidates at which the batch's pieces number at most the grid: from the
+// even share of all tiles (exact when the lengths are equal: the host's own
+// cut) towards the bound that always fits.  Each wavefront computes it for
+// itself, lane l holding sequence l (at most 64), without barriers.
 struct RaggedPiece {
     int b, u, piece, pieces, first;  // first: the workgroup of the segment's piece 0
     int2 v;                          // the sequence's (length, q position)
@@ -253,6 +252,7 @@ __device__ __forceinline__ RaggedPiece ragged_piece(const DecodeArgs& a, int U, 
     return r;
 }
 
+// Extent of sequence b as seen by one thread (no uniformity assumed).
 template <bool ALIGNED>
 __device__ __forceinline__ Extent lane_extent(const DecodeArgs& a, int b) {
     return extent_of<ALIGNED>(a, seq_values(a, b));
