@@ -8,6 +8,7 @@ device is not a gfx950, every call raises NyionError.
 from __future__ import annotations
 
 import ctypes as C
+import operator
 import os
 import struct
 
@@ -788,9 +789,10 @@ assert _GEMV_SPEC.size == C.sizeof(GemvSpec)
 
 def gemv_specs(specs, stream=None):
     """specs: list of (w, x, out, n_rows, n_cols, block_bytes) with device tensors."""
-    # packed as GemvSpec lays them out (ctypes structures cost 1 us each to fill)
-    m = 0xFFFFFFFF
-    arr = b"".join([_GEMV_SPEC.pack(ptr(w) or 0, ptr(x) or 0, ptr(out) or 0, nr & m, nc & m, bb & m, 0)
+    # packed as GemvSpec lays them out (ctypes structures cost 1 us each to
+    # fill), with whole numbers of any type, numpy's among them, as they take
+    m, i = 0xFFFFFFFF, operator.index
+    arr = b"".join([_GEMV_SPEC.pack(ptr(w) or 0, ptr(x) or 0, ptr(out) or 0, i(nr) & m, i(nc) & m, i(bb) & m, 0)
                     for w, x, out, nr, nc, bb in specs])
     check(load().nyion_gemv_specs(arr, len(specs), stream_handle(stream)), "nyion_gemv_specs")
 

@@ -5,6 +5,10 @@ import ctypes as C
 import os
 import re
 
+import numpy as np
+import pytest
+import torch
+
 import nyion_hip
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -84,3 +88,26 @@ def test_node_scratch_fits_the_reference_scores_buffer():
                 seen_split |= used > 0
     assert seen_split
     assert L.nyion_attention_node_scratch_bytes(30, 4, 128, 64) == 0  # invalid heads
+
+
+@pytest.mark.parametrize("whole", [int, np.int32, np.int64, np.uint8, lambda v: torch.tensor(v, dtype=torch.int32)])
+def test_gemv_specs_take_whole_numbers_of_any_type(monkeypatch, whole):
+    """The binding hands the library the bytes of GemvSpec, whatever type the
+    rows, columns and block bytes are held in (no device needed)."""
+    class Buffer:
+        def data_ptr(self):
+            return 0x1234567890
+
+    class Library:
+        def nyion_gemv_specs(self, arr, n, stream):
+            self.got = (bytes(arr), n)
+            return nyion_hip.OK
+
+    lib = Library()
+    monkeypatch.setattr(nyion_hip, "load", lambda: lib)
+    monkeypatch.setattr(nyion_hip, "stream_handle", lambda stream: None)
+    nyion_hip.gemv_specs([(Buffer(), None, Buffer(), whole(7), whole(64), whole(144))] * 2)
+    spec = bytes(nyion_hip.GemvSpec(0x1234567890, None, 0x1234567890, 7, 64, 144, 0))
+    assert lib.got == (2 * spec, 2)
+    with pytest.raises(TypeError):
+        nyion_hip.gemv_specs([(Buffer(), None, Buffer(), 7.0, 64, 144)])
