@@ -34,6 +34,7 @@
 // fp16 for P and V keeps 11 significant bits (p <= 2^14 after the lazy max),
 // so the P.V product stays within the f32 reference's tolerance; V must lie
 // within the fp16 range (|v| <= 65504).
+#include <limits.h>
 #include <math.h>
 
 #include <algorithm>
@@ -67,13 +68,15 @@ struct PrefillArgs {
     int n_items;   // kv heads x head subsets x row-block groups
     int causal;
     float scale_log2;
-    // the chunk's paged K/V write, done by the kernel (kv_write != 0): each
-    // workgroup of head subset 0 writes its own tokens' rows for its kv head
-    // after its attention work
+    // the chunk's paged K/V write, done by the kernel (kv_write == 0, no
+    // pools: only the range check of its V): by the workgroups from attn_wgs
+    // on, or (own_write) each workgroup of head subset 0 its own tokens' rows
+    // for its kv head after its attention work
     WriteArgs kvw;
     int kv_write;
     int kv_dtype;
-    int v_check;  // no pools: the same workgroups only check their V rows' range
+    int own_write;
+    int attn_wgs;
 };
 
 constexpr int BN = 64;  // keys per tile
@@ -262,30 +265,60 @@ __device__ __forceinline__ void stage_store_v(const VStage<D, NT>& st, unsigned 
     }
 }
 
-// A workgroup's share of the chunk's K/V rows, the tokens of its row blocks
-// for its kv head g, into the paged pools (every (token, kv head) by exactly
-// one workgroup), with the V range check the binary16 P.V product needs;
-// without pools, the check alone.
+// Items first, first + step, ... < end of the chunk's K/V rows (`at` gives an
+// item's row, kv head and four values) into the paged pools, with the V range
+// check the binary16 P.V product needs; without pools, the check alone.
+template <int D, class At>
+__device__ __forceinline__ void write_items(const PrefillArgs& a, int first, int end, int step, At at) {
+    float vmax = 0.f;
+    auto each = [&](auto write) __attribute__((always_inline)) {
+        for (int i = first; i < end; i += step) {
+            int r, g, x;
+            at(i, r, g, x);
+            vmax = fmaxf(vmax, write(r, g, x));
+        }
+    };
+    if (!a.kv_write)
+        each([&](int r, int g, int x) {
+            return v_absmax(*(const uint2*)(a.v + ((long long)r * a.n_kv_heads + g) * D + 4 * x));
+        });
+    else if (a.kv_dtype == NYION_KV_Q4_20B)  // 8 lanes per group: D / 4 is a multiple
+        each([&](int r, int g, int x) { return write_kv_q4_vec(a.kvw, r, g, x); });
+    else if (a.kv_dtype == NYION_KV_F16)
+        each([&](int r, int g, int x) { return write_kv_vec<true>(a.kvw, r, g, x); });
+    else
+        each([&](int r, int g, int x) { return write_kv_vec<false>(a.kvw, r, g, x); });
+    report_range(a.kvw.status, vmax >= 65520.f, kRangePrefillV);
+}
+
+// A workgroup's share of the write: the tokens of its row blocks for its kv
+// head g (every (token, kv head) by exactly one workgroup).
 template <int D>
 __device__ __forceinline__ void write_chunk_rows(const PrefillArgs& a, int g, int hs, int rbg, int tid,
                                                  int threads) {
-    if ((!a.kv_write && !a.v_check) || hs != 0) return;
+    if (!a.own_write || hs != 0) return;
     constexpr int VEC = D / 4;
     const int r0 = rbg * a.rb_per_wg * 32;
     const int r1 = min(a.n, r0 + a.rb_per_wg * 32);
-    float vmax = 0.f;
-    auto each = [&](auto write) __attribute__((always_inline)) {
-        for (int i = tid; i < (r1 - r0) * VEC; i += threads) vmax = fmaxf(vmax, write(r0 + i / VEC, i % VEC));
-    };
-    if (!a.kv_write)
-        each([&](int r, int x) { return v_absmax(*(const uint2*)(a.v + ((long long)r * a.n_kv_heads + g) * D + 4 * x)); });
-    else if (a.kv_dtype == NYION_KV_Q4_20B)
-        each([&](int r, int x) { return write_kv_q4_vec(a.kvw, r, g, x); });  // 8 lanes per group: VEC is a multiple
-    else if (a.kv_dtype == NYION_KV_F16)
-        each([&](int r, int x) { return write_kv_vec<true>(a.kvw, r, g, x); });
-    else
-        each([&](int r, int x) { return write_kv_vec<false>(a.kvw, r, g, x); });
-    report_range(a.kvw.status, vmax >= 65520.f, kRangePrefillV);
+    write_items<D>(a, tid, (r1 - r0) * VEC, threads, [&](int i, int& r, int& gi, int& x) {
+        r = r0 + i / VEC;
+        gi = g;
+        x = i % VEC;
+    });
+}
+
+// The whole write (of launches small enough for 32-bit item numbers), by the
+// workgroups behind the first a.attn_wgs.
+template <int D>
+__device__ __forceinline__ void write_chunk_apart(const PrefillArgs& a, int wg, int wgs, int tid, int threads) {
+    constexpr int VEC = D / 4;
+    write_items<D>(a, wg * threads + tid, a.n * a.n_kv_heads * VEC, wgs * threads,
+                   [&](int i, int& r, int& g, int& x) {
+                       const int row = i / VEC;
+                       r = row / a.n_kv_heads;
+                       g = row - r * a.n_kv_heads;
+                       x = i % VEC;
+                   });
 }
 
 template <int D>
@@ -304,6 +337,10 @@ __global__ __launch_bounds__(prefill_threads<D>(), 512 / prefill_threads<D>()) v
     const int j = lane & 31;   // row (S^T col) / dim within tile (O col)
     const int h = lane >> 5;   // half
 
+    if ((int)blockIdx.x >= a.attn_wgs) {
+        write_chunk_apart<D>(a, (int)blockIdx.x - a.attn_wgs, (int)gridDim.x - a.attn_wgs, tid, prefill_threads<D>());
+        return;
+    }
     // workgroup -> work item: XCD x = id % 8 takes items [x*per, (x+1)*per)
     const int per = (a.n_items + 7) / 8;
     const int item = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
@@ -879,7 +916,26 @@ static int launch_prefill(PrefillArgs& a, hipStream_t st, bool& split) {
     const long long items = prefill_items(a, prefill_threads<D>() / 64);
     if (items > (1LL << 30)) return set_error(NYION_ERR_UNSUPPORTED, "prefill: %lld work items", items);
     a.n_items = (int)items;
-    hipLaunchKernelGGL(prefill_kernel<D>, dim3(8 * ((a.n_items + 7) / 8)), dim3(prefill_threads<D>()), 0, st, a);
+    constexpr int threads = prefill_threads<D>();
+    int wgs = 8 * ((a.n_items + 7) / 8);
+    // The write of the chunk's rows by workgroups of its own where idle CUs
+    // hold enough of them to take fewer turns than the attention's workgroups
+    // would, one after the other: a turn of 4-bit rows is 0.5 us of arithmetic
+    // for the four wavefronts of a CU, one of f32 rows 0.3.  Measured (us, the
+    // attention's workgroups / apart / as a launch of its own): 4-bit pools,
+    // 12/12 heads of 64, 256 rows 17.7 / 9.3 / 13.6 and 400 rows 19.6 / 11.2 /
+    // 15.9; 32/8 heads of 128, 68 rows 14.5 / 9.1 / 13.3; 32/4 of 64, 33 rows
+    // 8.0 / 5.9 / 10.1; f32 pools, the same in turn 13.4 / 9.4, 15.6 / 11.4,
+    // 11.3 / 9.1 and 6.9 / 5.9.
+    const long long turns = (a.rb_per_wg * 32 * (D / 4) + threads - 1) / threads;
+    const long long needed = ((long long)a.n * a.n_kv_heads * (D / 4) + threads - 1) / threads;
+    const int idle = device_cu_count() - wgs;
+    if (idle > 0 && (needed + idle - 1) / idle < turns) {
+        a.own_write = 0;
+        a.attn_wgs = wgs;
+        wgs += (int)std::min<long long>(needed, idle);
+    }
+    hipLaunchKernelGGL(prefill_kernel<D>, dim3(wgs), dim3(threads), 0, st, a);
     return check_launch("prefill");
 }
 
@@ -924,6 +980,8 @@ static int prefill_impl(const uint16_t* q, const uint16_t* k, const uint16_t* v,
     a.n_kv_heads = n_kv_heads;
     a.group = group;
     a.causal = causal ? 1 : 0;
+    a.own_write = 1;
+    a.attn_wgs = INT_MAX;
     const float sc = scale > 0.f ? scale : 1.0f / sqrtf((float)head_dim);
     a.scale_log2 = sc * 1.4426950408889634f;
     if (k_pool || v_pool) {
@@ -935,7 +993,6 @@ static int prefill_impl(const uint16_t* q, const uint16_t* k, const uint16_t* v,
         a.kv_write = 1;
         a.kv_dtype = kv_dtype;
     } else {
-        a.v_check = 1;
         a.kvw.status = device_status_word();
     }
     hipStream_t st = (hipStream_t)stream;

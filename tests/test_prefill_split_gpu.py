@@ -94,3 +94,37 @@ def test_prefill_v_beyond_binary16_is_reported(gpu, where, d, n, hq):
         v[at, hkv - 1, d - 1] = big
         run_prefill_ctx(gpu, q[n_hist:], k[n_hist:], v[n_hist:], k[:n_hist], v[:n_hist])
         assert gpu.take_status()[0] == code, big
+
+
+# rows written by workgroups of their own, in one turn and in two (431), the
+# last turn partly used; and at 449 and 193 rows the first that the split
+# kernel's workgroups write
+@pytest.mark.parametrize("n,hq,hkv,d", [(1, 4, 4, 64), (33, 12, 12, 64), (256, 12, 12, 64), (431, 12, 12, 64), (449, 12, 12, 64),
+                                        (5, 8, 1, 64), (300, 32, 4, 64), (1, 2, 2, 128), (68, 32, 8, 128),
+                                        (130, 8, 8, 128), (192, 8, 8, 128), (193, 8, 8, 128)])
+def test_short_prefill_writes_and_checks_each_row_once(gpu, n, hq, hkv, d):
+    """Every row of a chunk without history, byte for byte what the K/V write
+    entry point stores, in each format; other rows keep their bytes.  Without
+    pools the V of the same rows is checked."""
+    bt, start = 16, 21
+    q, k, v = W.prefill_inputs(n, hq, hkv, d, seed=n + d)
+    nb = (start + n + bt - 1) // bt + 2
+    table = torch.from_numpy(np.random.default_rng(3).permutation(nb).astype(np.int32)).cuda()
+    rounded = [torch.from_numpy(W.bf16_round(x)).cuda() for x in (k, v)]
+    rows = np.unique(np.concatenate([np.arange(min(n, 20)), np.arange(max(0, n - 20), n)]))
+    ref = oracle_rows(q, k, v, rows)
+    for kv, row in ((oracle.KV_F32, 4 * d), (oracle.KV_F16, 2 * d), (oracle.KV_Q4, oracle.q4_row_bytes(d))):
+        got = [torch.full((nb, hkv, bt, row), 7, dtype=torch.uint8, device="cuda") for _ in "kv"]
+        want = [x.clone() for x in got]
+        gpu.kv_write(*want, table, bt, hkv, d, kv, start, *rounded)
+        check(run_prefill(gpu, q, k, v, k_pool=got[0], v_pool=got[1], block_table=table, block_tokens=bt,
+                          kv_dtype=kv, start_pos=start), ref, rows, f"{n} {hq}/{hkv} {d}")
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), kv
+    for at, h, x in ((0, 0, 0), (n - 1, hkv - 1, d - 1)):
+        big = v.copy()
+        big[at, h, x] = 65280.0
+        run_prefill(gpu, q, k, big)
+        assert gpu.take_status()[0] == 0
+        big[at, h, x] = -65536.0
+        run_prefill(gpu, q, k, big)
+        assert gpu.take_status()[0] == gpu.ERR_RANGE
