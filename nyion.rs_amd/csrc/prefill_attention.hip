@@ -901,17 +901,18 @@ template <int D>
 static int launch_prefill(PrefillArgs& a, hipStream_t st, bool& split) {
     constexpr int GW = D == 64 ? 2 : 4, NG = D == 64 ? 4 : 2;
     // Keys split over a workgroup's groups where one such workgroup per CU
-    // holds the launch and every group has two tiles to pipeline.  Measured
-    // (us, whole kernel / split): 32/4 heads of 64, 480 rows 13.3 / 12.6, 384
-    // rows 11.4 / 11.7, 640 rows (320 workgroups, two rounds) 15.3 / 18.1;
-    // 12/12 heads, 768 rows 18.7 / 13.6; 32/8 heads of 128, 256 rows 15.2 /
-    // 14.5, 64 rows 9.8 / 11.4, 1024 rows 34.0 / 27.5, 2048 rows after 2048
-    // 123 / 129; 512 rows after 1536 37.0 / 21.7 (d 64) and 59.0 / 43.3 (d
-    // 128).  With a history the split kernel also saves the launch that
-    // checks its V, which outweighs the merge at any length: one row after
-    // 128 12.5 / 9.7 (d 64) and 13.4 / 10.2 (d 128).
+    // holds the launch and there are tiles enough to pipeline.  Measured (us,
+    // whole kernel / split): 32/4 heads of 64, 384 rows 11.1 / 11.7, 450 rows
+    // 12.1 / 12.2, 512 rows 13.1 / 12.3, 640 rows (320 workgroups, two rounds)
+    // 15.3 / 18.1; 12/12 heads, 450 rows 13.3 / 12.6, 768 rows 17.7 / 15.0;
+    // 32/8 heads of 128, 256 rows 14.9 / 15.5, 320 rows 16.7 / 16.7, 384 rows
+    // 18.4 / 17.9, 1024 rows 37.3 / 29.4, 2048 rows after 2048 123 / 129; 512
+    // rows after 1536 37.0 / 21.7 (d 64) and 59.0 / 43.3 (d 128); into 4-bit
+    // pools the lines cross about 60 rows later.  With a history the split
+    // kernel also saves the launch that checks its V, which outweighs the merge
+    // at any length: one row after 128 12.5 / 9.7 (d 64) and 13.4 / 10.2 (d 128).
     const int tiles = (a.n_hist + BN - 1) / BN + (a.n + BN - 1) / BN;
-    split = prefill_items(a, GW) <= device_cu_count() && (tiles >= 2 * NG || a.n_hist > 0);
+    split = prefill_items(a, GW) <= device_cu_count() && (tiles >= (D == 64 ? 8 : 6) || a.n_hist > 0);
     if (split) return launch_prefill_split<D, GW, NG>(a, st);
     const long long items = prefill_items(a, prefill_threads<D>() / 64);
     if (items > (1LL << 30)) return set_error(NYION_ERR_UNSUPPORTED, "prefill: %lld work items", items);

@@ -25,6 +25,7 @@ CASES = [(0, 449, 4, 1, 64, True), (0, 513, 4, 4, 64, True), (0, 448, 4, 2, 64, 
          (1, 1, 4, 2, 64, True), (64, 1, 2, 1, 64, False), (129, 33, 6, 2, 64, True),
          (300, 77, 12, 12, 64, True), (575, 65, 8, 1, 64, False), (70, 512, 32, 4, 64, True),
          (70, 513, 32, 4, 64, True), (0, 193, 8, 2, 128, True), (0, 192, 8, 8, 128, False),
+         (0, 321, 8, 2, 128, True), (0, 385, 8, 8, 128, False),
          (1, 1, 4, 2, 128, True), (65, 31, 6, 3, 128, True), (190, 130, 8, 1, 128, False),
          (64, 257, 5, 5, 128, True), (100, 1024, 32, 8, 128, True), (100, 1025, 32, 8, 128, True)]
 
@@ -97,11 +98,11 @@ def test_prefill_v_beyond_binary16_is_reported(gpu, where, d, n, hq):
 
 
 # rows written by workgroups of their own, in one turn and in two (431), the
-# last turn partly used; and at 449 and 193 rows the first that the split
+# last turn partly used; and at 449 and 321 rows the first that the split
 # kernel's workgroups write
 @pytest.mark.parametrize("n,hq,hkv,d", [(1, 4, 4, 64), (33, 12, 12, 64), (256, 12, 12, 64), (431, 12, 12, 64), (449, 12, 12, 64),
                                         (5, 8, 1, 64), (300, 32, 4, 64), (1, 2, 2, 128), (68, 32, 8, 128),
-                                        (130, 8, 8, 128), (192, 8, 8, 128), (193, 8, 8, 128)])
+                                        (130, 8, 8, 128), (320, 8, 8, 128), (321, 8, 8, 128)])
 def test_short_prefill_writes_and_checks_each_row_once(gpu, n, hq, hkv, d):
     """Every row of a chunk without history, byte for byte what the K/V write
     entry point stores, in each format; other rows keep their bytes.  Without
