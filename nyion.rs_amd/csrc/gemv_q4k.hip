@@ -292,7 +292,8 @@ struct GemvSplitArgs {
     GemvMat mat[kGemvMaxMats];
     int units;       // of all matrices
     int full, rest;  // groups of blocks per wavefront, one more for the first `rest`
-    int waves;       // of a workgroup
+    int waves;       // of a workgroup that multiply
+    int converters;  // of a workgroup that convert the inputs (SHARED)
     const float* x;  // [n_inputs][x_stride]
     long long x_stride;
     long long out_stride;
@@ -315,9 +316,11 @@ __host__ __device__ constexpr int split_lds_bytes(int blocks, int nb, int B, int
 // R / 2 inputs for each of these blocks (the products of a block's weights
 // with another block's inputs are not used).
 //
-// The inputs are converted once per workgroup, or (EACH_STEP, for rows whose
-// operands would not fit the LDS) by each wavefront for each of its steps.
-template <int B, int R, bool EACH_STEP>
+// The inputs are converted once per workgroup, each wavefront's blocks by
+// itself or (SHARED: workgroups of one unit) all blocks by those that multiply
+// and more that only convert; or (EACH_STEP, for rows whose operands would not
+// fit the LDS) by each wavefront for each of its steps.
+template <int B, int R, bool EACH_STEP, bool SHARED>
 __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int KB = 16 / R;  // blocks per step
@@ -395,6 +398,30 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
     if constexpr (EACH_STEP) {
         load_step_x(0);
         load_w(first, 0, raw[0]);
+    } else if constexpr (SHARED) {
+        // all blocks' pairs among all wavefronts; the fence as below
+        auto item = [&](int i) __attribute__((always_inline)) { return (unsigned)min(2 * i + half, nb * B - 1); };
+        const int items = (nb * B + 1) / 2, di = a.converters;
+        auto load_at = [&](int i) __attribute__((always_inline)) {
+            const unsigned c = item(i);
+            return load_pair(c / B, c % B);
+        };
+        XShare cur = load_at(kp), next;
+        if (kp + di < items) next = load_at(kp + di);
+        asm volatile("" ::: "memory");
+        if (kp < P) load_w(first, 0, raw[0]);
+        for (int i = kp;;) {
+            const unsigned c = item(i);
+            store_pair(cur, lds + c / B * kBlk, c % B);
+            if ((i += di) >= items) break;
+            cur = next;
+            if (i + di < items) next = load_at(i + di);
+        }
+        __syncthreads();
+        if (kp >= P) {
+            __syncthreads();  // the unit's
+            return;
+        }
     } else {
         // all of this wavefront's blocks; the first weights are requested
         // behind the loads of the first pairs and ahead of their conversion.
@@ -787,12 +814,22 @@ static int launch_split_br(GemvSplitArgs& a, int cus, hipStream_t st) {
     a.waves = sh.waves;
     a.full = groups / sh.waves;
     a.rest = groups % sh.waves;
+    // Where a workgroup has one unit and no SIMD more than one wavefront that
+    // multiplies, the conversion is most of the launch, and more wavefronts
+    // share it: four inputs of 2048, 256 rows 4.7 -> 4.0 us, 2048 rows 5.2 ->
+    // 4.6, two inputs 3.7 -> 3.5.  With eight that multiply (1024 x 4096, four
+    // inputs) 6.2 -> 6.3.
+    a.converters = sh.waves;
+    if (B > 1 && !sh.each_step && units <= cus && sh.waves <= 4)
+        a.converters = std::max(sh.waves, std::min(16, ceil_div(a.nb * B, 2)));
+    const bool shared = a.converters > sh.waves;
     // resident workgroups: four or (one input) five wavefronts per SIMD
     const int cap = std::max(1, std::min((B > 1 ? 16 : 20) / sh.waves, kLdsPerCu / sh.lds)) * cus;
-    static std::atomic<int> allowed[2][kMaxDevices];
-    auto kernel = sh.each_step ? gemv_split_kernel<B, R, true> : gemv_split_kernel<B, R, false>;
-    allow_lds(allowed[sh.each_step], kernel, sh.lds);
-    hipLaunchKernelGGL(kernel, dim3(std::min(units, cap)), dim3(64 * sh.waves), sh.lds, st, a);
+    static std::atomic<int> allowed[3][kMaxDevices];
+    auto kernel = sh.each_step ? gemv_split_kernel<B, R, true, false> : gemv_split_kernel<B, R, false, false>;
+    if (shared) kernel = gemv_split_kernel<B, R, false, (B > 1)>;
+    allow_lds(allowed[shared ? 2 : sh.each_step], kernel, sh.lds);
+    hipLaunchKernelGGL(kernel, dim3(std::min(units, cap)), dim3(64 * a.converters), sh.lds, st, a);
     return check_launch("gemv q4k");
 }
 

@@ -26,6 +26,10 @@ CASES = [
     (65, 2304, 17), (129, 512, 33), (383, 1280, 31), (385, 256, 100), (2050, 512, 200),
     (40, 5632, 6), (40, 5632, 13), (24, 14336, 1), (24, 14336, 3), (24, 14336, 7),
     (9, 53248, 2), (9, 53248, 1),
+    # inputs converted by wavefronts that do not multiply: fewer pairs than
+    # wavefronts, an odd number, more than one turn; the last row count and
+    # length that take it, and the next
+    (7, 256, 3), (40, 768, 2), (65, 1280, 4), (2048, 2048, 4), (2049, 2048, 3), (16, 2304, 4), (30, 1024, 7),
 ]
 
 
