@@ -1330,7 +1330,8 @@ constexpr bool span_tiles() {
 // NB - 1 ahead.  A Q4-20B span tile is 1280 bytes at head_dim 64, a sixth of
 // an f32 tile, so it takes a ring of four; at head_dim 128 too, except for
 // tracked walks, whose scores leave no registers for it (4 sequences of
-// 3000-9000 tokens: per-row loads 33.8 us, a ring of two 28.9, of four 39.5).
+// 3000-9000 tokens: per-row loads 33.8 us, a ring of two 28.9, of four 39.5;
+// with two, the stream-K kernel still keeps 8 registers in scratch).
 // Gathered tiles (position lists, strided globals) keep two: their walks are
 // short, and the extra tiles loaded past a walk's end cost more than the
 // deeper ring gains.
@@ -1662,9 +1663,10 @@ __device__ __forceinline__ int sload(const int* p) { return __builtin_amdgcn_rea
 // register-resident 16-token tiles alone take 128 VGPRs per lane (one), and
 // the smaller binary16 tiles at head_dim 64 (three).  Two tiles of loads in
 // flight per wavefront at this occupancy keep ~32 MB of f32 reads
-// outstanding, more than HBM latency x bandwidth.  The 4-bit kernels keep
-// two: at three their binary16 products spill, and the 131072-token window
-// runs 10 % faster at two.
+// outstanding, more than HBM latency x bandwidth.  The 4-bit kernels and
+// binary16 at head_dim 128 keep two: at three they spill 11 to 131 registers
+// (8 windows of 4096 tokens: 4-bit 15.5 -> 20.9 us at head_dim 64 and 23.6 ->
+// 44.3 at 128, binary16 32.8 -> 52.6).
 template <int D, int KVT>
 constexpr int decode_waves_per_eu() {
     return (D == 128 && KVT == NYION_KV_F32) ? 1 : (D == 64 && KVT == NYION_KV_F16) ? 3 : 2;
@@ -2327,7 +2329,9 @@ constexpr long long kRaggedMaxBytes = 200LL << 20;
 // partials.  The pieces are then raised to one workgroup per CU where each
 // keeps kDirectMinPieceTiles tiles: with the CUs otherwise idle, the
 // shorter walks gain more than the extra partials cost (8 windows of 4096
-// tokens, 4 kv heads: 128 -> 256 workgroups, 14.8 -> 13.5 us).  The tuning
+// tokens, 4 kv heads: 128 -> 256 workgroups, 14.8 -> 13.5 us).  Half or twice
+// of each of the three leaves the geometric mean of 275 decode launches of all
+// formats within 0.4 %, single ones moving up to 25 % either way.  The tuning
 // override, when set, is used as it is.
 constexpr long long kDirectWgBytes = 96 << 10;
 constexpr long long kDirectMinGrid = 128;

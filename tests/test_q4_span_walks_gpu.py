@@ -87,9 +87,8 @@ def test_q4_span_walk_tracked(gpu, tokens):
 def test_q4_attention_node(gpu, head_dim, seq_len):
     """The Attention node on Q4-20B rows laid out [Hkv][kv_stride][row]
     (compute_graph.rs:14-25 with the 4-bit cache): no block table, so a span
-    walk's tile offsets come from the row positions alone (head_dim 64;
-    head_dim 128 walks per-row tiles), with and without the scores buffer
-    (whole segments, or split-K pieces merged through it)."""
+    walk's tile offsets come from the row positions alone, with and without the
+    scores buffer (whole segments, or split-K pieces merged through it)."""
     rng = np.random.default_rng(seq_len + head_dim)
     hq, hkv, stride = 32, 4, seq_len + 24
     q = rng.standard_normal((hq, head_dim), dtype=np.float32)
