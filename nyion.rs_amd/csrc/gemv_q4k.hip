@@ -38,13 +38,14 @@
 // gemv_tile_kernel (more): the wavefronts take different rows and walk the
 // blocks together over inputs converted once per workgroup.
 //
-// What bounds them.  Up to eight inputs, HBM: a wavefront's 16 rows x 256
-// weights are 2304 bytes, 130 VALU instructions (88 of them for the weights,
-// half at half rate) and 12 MFMAs, where a convert and an FMA per weight and
-// input were 300 instructions for the first input alone.  Many inputs, VALU
-// and matrix cores about equally.  Before and after, us: 14336 x 4096, one
-// input 12.8 and 10.9, eight inputs 65.8 and 15.6; 5632 x 2048, 509 inputs
-// 1320 and 39.
+// What bounds them.  Up to eight inputs, HBM and the chain in front of it: a
+// wavefront's 16 rows x 256 weights are 2304 bytes, 125 VALU instructions (143
+// with eight inputs) and 11 MFMAs, where a convert and an FMA per weight and
+// input were 300 instructions for the first input alone; 14336 x 4096 with
+// eight inputs keeps the VALU 63 % and the matrix cores 8 % busy.  Many inputs,
+// VALU and matrix cores in turn: 5632 x 2048 with 509 inputs 65 % and 32 %.
+// f32 FMAs and now, us: 14336 x 4096, one input 12.8 and 9.7, eight inputs 65.7
+// and 14.6; 5632 x 2048, 509 inputs 1318 and 40.9.
 #include "gemv.hpp"
 
 #include <limits.h>
