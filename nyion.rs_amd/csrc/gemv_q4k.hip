@@ -27,9 +27,9 @@
 // A block's value for one (row, input) is a chain of eight K steps, and an
 // output is the sum of kSumWays sums of its blocks' values, whichever kernel,
 // tile or wavefront computed them: single, multi-matrix and batched calls
-// give the same bits.  Against float64 the outputs are off by 1.6e-7 to 1.8e-7
-// of their norm for N(0, 1) inputs (256 to 14336 columns; f32 FMAs in runs of
-// 16 were 1.8e-7 to 2.1e-7), and as much beside a value 2^28 times the others
+// give the same bits.  Against float64 the outputs are off by 1.5e-7 to 1.8e-7
+// of their norm for N(0, 1) inputs (512 to 14336 columns; f32 FMAs in runs of
+// 16 were 1.5e-7 to 2.2e-7), and as much beside a value 2^28 times the others
 // that meets zero weights.
 //
 // Two kernels.  gemv_split_kernel (up to eight inputs): the wavefronts of a
@@ -40,7 +40,7 @@
 //
 // What bounds them.  Up to eight inputs, HBM and the chain in front of it: a
 // wavefront's 16 rows x 256 weights are 2304 bytes, 125 VALU instructions (143
-// with eight inputs) and 11 MFMAs, where a convert and an FMA per weight and
+// with eight inputs) and 10 MFMAs, where a convert and an FMA per weight and
 // input were 300 instructions for the first input alone; 14336 x 4096 with
 // eight inputs keeps the VALU 63 % and the matrix cores 8 % busy.  Many inputs,
 // VALU and matrix cores in turn: 5632 x 2048 with 509 inputs 65 % and 32 %.
@@ -268,8 +268,8 @@ __device__ __forceinline__ floatx4 mfma(const halfx8& a, const halfx8& b, const 
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-// Operands of the products with a word per lane on either side (the sums of x
-// per sub-block): the other three words stay zero in their registers.  (The
+// Operands of the products with a word or two per lane on either side (the
+// sums of x per sub-block): the other words stay zero in their registers.  (The
 // K = 16 form, of half the words, gave wrong sums behind a K = 32 chain into
 // the same accumulator with this compiler.)
 __device__ __forceinline__ u32x4 zero_words() {
@@ -498,15 +498,17 @@ __global__ __launch_bounds__(1024) void gemv_split_kernel(GemvSplitArgs a) {
             const halfx8 xv = as_half8(*(const u32x4*)(op0 + off + st * 128 * B));
             acc = mfma(xv, Q4k::weights(cur, sc, st), acc);
         }
-        // the offsets' term as the weights' (hi and lo rows), the mins' in turn
-        // into the rows of hi
+        // the offsets' term as the weights' (hi and lo rows); the mins' with both
+        // terms of the sums of x, as two words, into the rows of hi: two products
+        // one after the other were off by 4 % more (1.7e-7) and took 1.5 % longer
+        // (14336 x 4096, eight inputs)
         word_a.x = *(const uint32_t*)(sum0 + off);
+        word_a.y = 0;
         word_b.x = sc.offsets;
-        word_c.x = sc.mins;
         acc = mfma(as_half8(word_a), as_half8(word_b), acc);
-        accm = mfma(as_half8(word_a), as_half8(word_c), accm);
-        word_a.x = *(const uint32_t*)(sum0 + off + 4 * B);
-        word_c.x = sc.mins_low;
+        word_a.y = *(const uint32_t*)(sum0 + off + 4 * B);
+        word_c.x = sc.mins;
+        word_c.y = sc.mins_low;
         accm = mfma(as_half8(word_a), as_half8(word_c), accm);
         float v[kRegs];
 #pragma unroll
@@ -603,7 +605,7 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
 #pragma unroll
     for (int i = 0; i < RT; i++) wp[i] = a.w + min(row0 + 16 * i + n, a.rows - 1) * row_bytes;
 
-    u32x4 word_h = zero_words(), word_l = zero_words(), word_w = zero_words();
+    u32x4 word_h = zero_words(), word_l = zero_words(), word_w = zero_words(), word_m = zero_words();
     floatx4 total[RT][MT];  // the sum in progress
 #pragma unroll
     for (int i = 0; i < RT; i++)
@@ -691,16 +693,15 @@ __global__ __launch_bounds__(64 * RW * KS, WPS) void gemv_tile_kernel(GemvTileAr
             for (int j = 0; j < MT; j++) {
                 const floatx4 inv = *(const floatx4*)&X.inv[16 * j + 4 * g];
                 word_h.x = X.sums[j][0][g][n];
-                word_l.x = X.sums[j][1][g][n];
+                word_h.y = word_l.x = X.sums[j][1][g][n];
 #pragma unroll
                 for (int i = 0; i < RT; i++) {
                     word_w.x = sc[i].offsets;
                     hi[i][j] = mfma(as_half8(word_h), as_half8(word_w), hi[i][j]);
                     lo[i][j] = mfma(as_half8(word_l), as_half8(word_w), lo[i][j]);
-                    word_w.x = sc[i].mins;
-                    floatx4 m = mfma(as_half8(word_h), as_half8(word_w), floatx4{0.f, 0.f, 0.f, 0.f});
-                    word_w.x = sc[i].mins_low;
-                    m = mfma(as_half8(word_l), as_half8(word_w), m);
+                    word_m.x = sc[i].mins;
+                    word_m.y = sc[i].mins_low;
+                    const floatx4 m = mfma(as_half8(word_h), as_half8(word_m), floatx4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                     for (int r = 0; r < 4; r++)
                         total[i][j][r] = __builtin_fmaf(
