@@ -42,10 +42,10 @@
 // wavefront's 16 rows x 256 weights are 2304 bytes, 125 VALU instructions (143
 // with eight inputs) and 10 MFMAs, where a convert and an FMA per weight and
 // input were 300 instructions for the first input alone; 14336 x 4096 with
-// eight inputs keeps the VALU 63 % and the matrix cores 8 % busy.  Many inputs,
-// VALU and matrix cores in turn: 5632 x 2048 with 509 inputs 65 % and 32 %.
+// eight inputs keeps the VALU 64 % and the matrix cores 7 % busy.  Many inputs,
+// VALU and matrix cores in turn: 5632 x 2048 with 509 inputs 65 % and 31 %.
 // f32 FMAs and now, us: 14336 x 4096, one input 12.8 and 9.7, eight inputs 65.7
-// and 14.6; 5632 x 2048, 509 inputs 1318 and 40.9.
+// and 14.6; 5632 x 2048, 509 inputs 1319 and 39.8.
 #include "gemv.hpp"
 
 #include <limits.h>
