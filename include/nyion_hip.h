@@ -96,6 +96,7 @@ int nyion_take_status(nyion_stream_t stream);
  * token at q_pos = seq_len-1: out[h] = softmax(q[h].K[kv(h)]^T / sqrt(D)) V,
  * kv(h) = h / (n_heads/n_kv_heads).
  * Layout: d_q, d_out [n_heads][head_dim] f32; d_k, d_v [n_kv_heads][kv_stride][row].
+ * Nothing behind the last head's kv_stride rows is read.
  * d_scores: optional f32 scratch of at least n_heads*seq_len floats (the
  * node's scores buffer: ScratchBuffers::d_scores holds n_heads*window_size,
  * swamp-gpu/src/lib.rs:317; the CUDA path n_heads*seq_len,
